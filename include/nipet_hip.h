@@ -93,6 +93,13 @@ int nipet_tx_lists(const NipetGeom *g, int64_t *offsets, int32_t *col, float *t,
 int nipet_fprj(const NipetGeom *g, float *sino, const float *img, const int32_t *subs, int nprj,
                int att, void *stream);
 
+/* nipet_fprj by segments: the same projections (they differ by 5e-8), every
+ * LOR visiting every segment of its ray in float32. The differentiable
+ * projectors' forward passes use it, so that the float64 likelihood made of
+ * these values keeps its bits. */
+int nipet_fprj_seg(const NipetGeom *g, float *sino, const float *img, const int32_t *subs,
+                   int nprj, int att, void *stream);
+
 /* Back projection (petprj.bprj, prj/src/prj_module.cu:430-608;
  * gpu_bprj prj/src/prjb.cu:190-308): img (device) is overwritten with the
  * adjoint of the emission projector applied to sino [nprj][nsn] (device). */

@@ -75,6 +75,7 @@ def lib():
             'nipet_geom_info': ([P, P, P, P, P], I),
             'nipet_tx_lists': ([P, P, P, P, P], I),
             'nipet_fprj': ([P, P, P, P, I, I, P], I),
+            'nipet_fprj_seg': ([P, P, P, P, I, I, P], I),
             'nipet_bprj': ([P, P, P, P, I, P], I),
             'nipet_osem_corr': ([P, P, P, P, P, P, I64, P], I),
             'nipet_osem_sens': ([P, P, P, P, I, P], I),

@@ -14,6 +14,7 @@ constexpr int NZ = 127;   // device image z (w), fastest
 // segments of one transaxial ray: one per voxel column it crosses, at most
 // one more than the grid lines it crosses (checked when the geometry is built)
 constexpr int MAX_SEG = NX + NY + 1;
+constexpr int SEG_PAD = 64;  // records behind the last list (whole chunks are read)
 constexpr int64_t NVOX = (int64_t)NX * NY * NZ;
 constexpr int MAXNSN = 4096;  // largest sinogram count handled (span-1: 4084)
 constexpr int LI_MAX = 2112;  // largest Michelogram (ring pair) count
@@ -29,6 +30,24 @@ struct __align__(16) SegRec {
   int32_t colz;
 };
 
+// What the kernels read of a geometry.
+struct GeomView {
+  const int32_t *off;
+  const SegRec *seg;
+  const double *atn;
+  const uint2 *ev;
+  const float *lmax;
+  const float2 *li_z;
+  const short2 *li_sn;
+  const float *li_nosi;
+  const int16_t *dr_li;
+  const uint16_t *sn_mem;
+  const uint16_t *bp_tab;
+  const int16_t *fp_slot;
+  int naw, nli, ndirect, nsn, dmax, sn_w, fp_nslot;
+  float vox_z;
+};
+
 // Geometry resident on one device. Transaxial intersection lists in CSR form:
 // segments of ray aw are seg[off[aw] .. off[aw+1]).
 struct Geom {
@@ -40,6 +59,11 @@ struct Geom {
   SegRec *seg = nullptr;     // [nseg]
   double *atn = nullptr;     // [naw] crystal-to-crystal transaxial distance
   float *lmax = nullptr;     // [naw] longest segment of the ray
+  // z crossings of a ray [naw][ev_off(dmax + 1)]: entry ev_off(d) + w is where
+  // the LORs of ring difference d pass from plane offset w to w + 1, at t =
+  // (w + 1/2) atn / (2 d): (segment << 10 | ev_phi(w), distance into the
+  // segment), segment 2^22 - 1 past the end of the list
+  uint2 *ev = nullptr;
   float2 *li_z = nullptr;    // [nli] (zeta_a at t=0, zeta_b - zeta_a) in z-voxel units
   short2 *li_sn = nullptr;   // [nli] output sinogram of LOR a and of its mirror b
   float *li_nosi = nullptr;  // [nli] 1 / (span-1 LORs per output sinogram)
@@ -47,10 +71,12 @@ struct Geom {
   // starts there) and ring r0 + d
   int dmax = 0;                // largest ring difference d
   int16_t *dr_li = nullptr;    // [64 * 64] li of (d, r0) at d * 64 + r0, -1 if absent
-  int32_t *sn_off = nullptr;   // [nsn + 1] CSR of the span-1 LORs of each output sinogram:
-  int16_t *sn_mem = nullptr;   // [2 nli] 2 li (LOR a) or 2 li + 1 (mirror b)
-  // forward-projector lane slots: slot s walks the LORs (d, r0 + k), k < FP_G,
-  // of one ring difference; fp_slot[s] = d * 64 + r0
+  // the span-1 LORs of each output sinogram [nsn][sn_w]: 2 li (LOR a) or
+  // 2 li + 1 (mirror b), 2 LI_MAX where there are fewer (span 11: at most 6)
+  uint16_t *sn_mem = nullptr;
+  int sn_w = 8;  // a multiple of 8
+  // segment-walking forward projector (k_fprj_seg): slot s walks the LORs
+  // (d, r0 + k), k < FP_G, of one ring difference; fp_slot[s] = d * 64 + r0
   int16_t *fp_slot = nullptr;
   int fp_nslot = 0;
   // back-projector LOR tables [3][2][BP_TABN] for 1, 2 and 4 images: byte
@@ -58,6 +84,8 @@ struct Geom {
   // LOR (r0, d) and of its mirror at bp_row(d) + d + 1 + r0; the zero row
   // (nsn * nb * 4) where there is none
   uint16_t *bp_tab = nullptr;
+  GeomView view = {};           // the pointers above, and
+  GeomView *dview = nullptr;    // its copy on the device
 };
 
 // Rows of the back projector's LOR tables: row d holds r0 = -d-1 .. 64
@@ -66,7 +94,14 @@ constexpr int BP_MAXD = 63;  // largest ring difference of the BP tables
 __host__ __device__ constexpr int bp_row(int d) { return 66 * d + d * (d - 1) / 2; }
 constexpr int BP_TABN = bp_row(BP_MAXD + 1);
 
-constexpr int FP_G = 3;          // LORs per forward-projector lane
+// Position of plane w in the forward projector's LDS rows (64 even planes, then
+// 64 odd ones, of 8 bytes), in bytes.
+__host__ __device__ constexpr int ev_phi(int w) { return ((w & 1) << 9) + ((w >> 1) << 3); }
+// Crossings of ring difference d in Geom::ev: 2 d, and eight that lie past any
+// segment (eight are read at a time).
+__host__ __device__ constexpr int ev_off(int d) { return (d - 1) * (d + 8); }
+
+constexpr int FP_G = 3;          // LORs per lane of k_fprj_seg
 constexpr int FP_G_SLOTS = 768;  // lanes of that kernel
 
 void set_error(const char *fmt, ...);

@@ -20,6 +20,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -234,6 +235,40 @@ __global__ void k_tx_lists(const float *crs, const short2 *s2c, int naw, double 
   }
 }
 
+// z crossings of every ray (Geom::ev), one workgroup per bin: a binary search
+// of t in the bin's segment starts per crossing. (Crossings before the list
+// get its start; no walk reads them.)
+__global__ __launch_bounds__(256) void k_events(const int32_t *__restrict__ off,
+                                                const SegRec *__restrict__ seg,
+                                                const double *__restrict__ atn, int dmax,
+                                                uint2 *__restrict__ ev) {
+  __shared__ double s[MAX_SEG];
+  const int aw = blockIdx.x, beg = off[aw], n = off[aw + 1] - beg;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) s[i] = seg[beg + i].s;
+  __syncthreads();
+  const int ne = ev_off(dmax + 1);
+  for (int i = threadIdx.x; i < ne; i += blockDim.x) {
+    int d = (int)sqrtf((float)i + 2.25f);  // ev_off(d) <= i < ev_off(d + 1)
+    while (ev_off(d) > i) d--;
+    while (ev_off(d + 1) <= i) d++;
+    const int w = i - ev_off(d);
+    const double t = ((double)w + 0.5) * (atn[aw] / (2.0 * d));
+    int lo = 0, hi = n;  // s[lo] <= t < s[hi]
+    while (hi - lo > 1) {
+      const int m = (lo + hi) >> 1;
+      if (s[m] <= t) lo = m; else hi = m;
+    }
+    uint2 e = make_uint2(~0u, 0u);
+    if (n > 0) {
+      const float len = seg[beg + lo].len;
+      if (w < 2 * d && (lo < n - 1 || t < s[lo] + (double)len))
+        e.x = ((unsigned)lo << 10) | (unsigned)ev_phi(w);
+      e.y = __float_as_uint(fminf(fmaxf((float)(t - s[lo]), 0.f), len));
+    }
+    ev[(size_t)aw * ne + i] = e;
+  }
+}
+
 // Bins of a subset ordered by decreasing segment count (bins outside
 // 0 .. naw-1 last), one workgroup: a counting sort by count with LDS buckets.
 // Bins of equal count keep no particular order: the order only decides which
@@ -310,7 +345,7 @@ int nipet_prof_read(int kernel, double *total_ms, int64_t *count) {
 static void geom_free(Geom *g) {
   // teardown: a failing free leaves nothing to undo
   void *bufs[] = {g->off,   g->seg,    g->atn,    g->lmax,   g->li_z,   g->li_sn,
-                  g->li_nosi, g->dr_li, g->sn_off, g->sn_mem, g->fp_slot, g->bp_tab};
+                  g->li_nosi, g->dr_li, g->sn_mem, g->fp_slot, g->bp_tab, g->ev, g->dview};
   for (void *p : bufs) (void)hipFree(p);
 }
 
@@ -359,8 +394,7 @@ static int geom_build(const NipetGeomDesc *d, NipetGeom *g) {
   // two z-voxels), so LOR a of li starts on ring r0 = (zeta_a - 0.5) / 2 and
   // spans d = (zeta_b - zeta_a) / 2 rings
   std::vector<int16_t> drli(64 * 64, -1);
-  std::vector<int32_t> snoff(d->nsn + 1, 0);
-  std::vector<int16_t> snmem;
+  std::vector<uint16_t> snmem;
   if (d->nli > LI_MAX) {
     set_error("more than %d Michelogram elements", LI_MAX);
     return NIPET_EINVAL;
@@ -380,18 +414,19 @@ static int geom_build(const NipetGeomDesc *d, NipetGeom *g) {
     drli[dd * 64 + r0] = (int16_t)li;
     g->dmax = dd > g->dmax ? dd : g->dmax;
   }
-  for (int li = 0; li < d->nli; li++) {
-    snoff[lisn[li].x + 1]++;
-    if (liz[li].y > 0.f) snoff[lisn[li].y + 1]++;
-  }
-  for (int s = 0; s < d->nsn; s++) snoff[s + 1] += snoff[s];
-  snmem.assign(snoff[d->nsn] > 0 ? snoff[d->nsn] : 1, 0);
   {
-    std::vector<int32_t> fill(snoff.begin(), snoff.end() - 1);
-    for (int li = 0; li < d->nli; li++) {
-      snmem[fill[lisn[li].x]++] = (int16_t)(2 * li);
-      if (liz[li].y > 0.f) snmem[fill[lisn[li].y]++] = (int16_t)(2 * li + 1);
-    }
+    std::vector<int> fill(d->nsn, 0);
+    auto members = [&](auto &&f) {
+      for (int li = 0; li < d->nli; li++) {
+        f(lisn[li].x, 2 * li);
+        if (liz[li].y > 0.f) f(lisn[li].y, 2 * li + 1);
+      }
+    };
+    members([&](int s, int) { fill[s]++; });
+    for (int s = 0; s < d->nsn; s++) g->sn_w = std::max(g->sn_w, (fill[s] + 7) / 8 * 8);
+    snmem.assign((size_t)d->nsn * g->sn_w, (uint16_t)(2 * LI_MAX));
+    fill.assign(d->nsn, 0);
+    members([&](int s, int m) { snmem[(size_t)s * g->sn_w + fill[s]++] = (uint16_t)m; });
   }
   // forward-projector slots: the LORs of one ring difference d in groups of
   // FP_G consecutive r0 (ordered by d, then r0); LOR (d, r0 + k) lies exactly
@@ -439,13 +474,10 @@ static int geom_build(const NipetGeomDesc *d, NipetGeom *g) {
                         hipMemcpyHostToDevice));
   }
   NIPET_HIP(hipMalloc(&g->dr_li, drli.size() * sizeof(int16_t)));
-  NIPET_HIP(hipMalloc(&g->sn_off, snoff.size() * sizeof(int32_t)));
-  NIPET_HIP(hipMalloc(&g->sn_mem, snmem.size() * sizeof(int16_t)));
+  NIPET_HIP(hipMalloc(&g->sn_mem, snmem.size() * sizeof(uint16_t)));
   NIPET_HIP(hipMemcpy(g->dr_li, drli.data(), drli.size() * sizeof(int16_t),
                       hipMemcpyHostToDevice));
-  NIPET_HIP(hipMemcpy(g->sn_off, snoff.data(), snoff.size() * sizeof(int32_t),
-                      hipMemcpyHostToDevice));
-  NIPET_HIP(hipMemcpy(g->sn_mem, snmem.data(), snmem.size() * sizeof(int16_t),
+  NIPET_HIP(hipMemcpy(g->sn_mem, snmem.data(), snmem.size() * sizeof(uint16_t),
                       hipMemcpyHostToDevice));
 
   NIPET_HIP(hipMalloc(&g->li_z, d->nli * sizeof(float2)));
@@ -507,10 +539,19 @@ static int geom_build(const NipetGeomDesc *d, NipetGeom *g) {
   }
   g->nseg = tot;
   NIPET_HIP(hipMemcpy(g->off, off.data(), (d->naw + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
-  NIPET_HIP(hipMalloc(&g->seg, (tot + 1) * sizeof(SegRec)));
+  // the projectors read whole chunks of records: padded behind the last list
+  NIPET_HIP(hipMalloc(&g->seg, (tot + SEG_PAD) * sizeof(SegRec)));
+  NIPET_HIP(hipMemset(g->seg + tot, 0, SEG_PAD * sizeof(SegRec)));
   k_tx_lists<<<nb, 256>>>(d_crs, d_s2c, d->naw, (double)d->vox_xy, (double)d->tfov2, NZ, g->off,
                           nullptr, g->seg, nullptr, g->lmax, d_err);
   NIPET_HIP(hipGetLastError());
+  if (g->dmax > 0) {  // eight crossings are read at a time
+    const size_t ne = ev_off(g->dmax + 1);
+    NIPET_HIP(hipMalloc(&g->ev, (d->naw * ne + 8) * sizeof(uint2)));
+    NIPET_HIP(hipMemset(g->ev + d->naw * ne, 0xff, 8 * sizeof(uint2)));
+    k_events<<<d->naw, 256>>>(g->off, g->seg, g->atn, g->dmax, g->ev);
+    NIPET_HIP(hipGetLastError());
+  }
   NIPET_HIP(hipDeviceSynchronize());
   // the projectors split a segment into at most three z pieces: no segment may
   // span two z-boundary spacings atn / (2 dmax) of the steepest LOR
@@ -525,6 +566,29 @@ static int geom_build(const NipetGeomDesc *d, NipetGeom *g) {
         return NIPET_EINVAL;
       }
   }
+  GeomView &v = g->view;
+  v.off = g->off;
+  v.seg = g->seg;
+  v.atn = g->atn;
+  v.ev = g->ev;
+  v.lmax = g->lmax;
+  v.li_z = g->li_z;
+  v.li_sn = g->li_sn;
+  v.li_nosi = g->li_nosi;
+  v.dr_li = g->dr_li;
+  v.sn_mem = g->sn_mem;
+  v.bp_tab = g->bp_tab;
+  v.fp_slot = g->fp_slot;
+  v.fp_nslot = g->fp_nslot;
+  v.naw = g->naw;
+  v.nli = g->nli;
+  v.ndirect = g->ndirect;
+  v.nsn = g->nsn;
+  v.dmax = g->dmax;
+  v.sn_w = g->sn_w;
+  v.vox_z = g->vox_z;
+  NIPET_HIP(hipMalloc(&g->dview, sizeof(GeomView)));
+  NIPET_HIP(hipMemcpy(g->dview, &v, sizeof(GeomView), hipMemcpyHostToDevice));
   return NIPET_OK;
 }
 

@@ -62,13 +62,15 @@ class Projector:
         self._s1map = None
 
     # -- raw kernels (no autograd) -------------------------------------------------
-    def fp(self, img, att=False, geom=None):
+    def fp(self, img, att=False, geom=None, name='nipet_fprj_seg'):
+        """Forward projection by segments (the float64 likelihood made of it
+        keeps its bits), or by z crossings with ``name='nipet_fprj'``."""
         torch = _torch()
         g = self.geom if geom is None else geom
         out = torch.empty((self.nprj, g.nsn), dtype=torch.float32, device=img.device)
-        _lib.check(_lib.lib().nipet_fprj(g.handle, _lib.ptr(out), _lib.ptr(img),
-                                         _lib.ptr(self.subs), self.nprj, int(bool(att)),
-                                         _lib.stream_handle()), 'nipet_fprj')
+        _lib.check(getattr(_lib.lib(), name)(g.handle, _lib.ptr(out), _lib.ptr(img),
+                                             _lib.ptr(self.subs), self.nprj, int(bool(att)),
+                                             _lib.stream_handle()), name)
         return out
 
     def bp(self, sino, geom=None):
@@ -105,7 +107,7 @@ class Projector:
     def attenuation_vjp(self, mu, g):
         """J^T g for a = attenuation_fp(mu): -A1^T(exp(-A1 mu) * g[b] / n_b)."""
         g1, s11, inv = self.span1()
-        t = self.fp(mu, att=False, geom=g1)           # span-1 line integrals (nprj, 4084)
+        t = self.fp(mu, geom=g1, name='nipet_fprj')   # span-1 line integrals (nprj, 4084)
         t.neg_().exp_()
         t.mul_(g.index_select(1, s11)).mul_(inv)
         return self.bp(t, geom=g1).neg_()
