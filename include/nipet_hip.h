@@ -93,6 +93,16 @@ int nipet_tx_lists(const NipetGeom *g, int64_t *offsets, int32_t *col, float *t,
 int nipet_fprj(const NipetGeom *g, float *sino, const float *img, const int32_t *subs, int nprj,
                int att, void *stream);
 
+/* Scratch of the calling thread's back projections (nipet_bprj*, nipet_osem_*):
+ * a device buffer, 256-byte aligned, that every later call of this thread may
+ * overwrite in its stream's order, until it is replaced or taken back with (NULL,
+ * 0). With at least nipet_bprj_scratch bytes the per-segment sums are staged
+ * there and gathered by voxel column (a fixed order of additions); with less, in
+ * several passes; without, or for few bins, they are float atomics into the
+ * image. nipet_bprj_scratch: bytes for nprj bins of nb images (0: none used). */
+int64_t nipet_bprj_scratch(const NipetGeom *g, int nprj, int nb);
+int nipet_scratch_set(void *buf, int64_t bytes);
+
 /* nipet_fprj by segments: the same projections (they differ by 5e-8), every
  * LOR visiting every segment of its ray in float32. The differentiable
  * projectors' forward passes use it, so that the float64 likelihood made of
@@ -427,9 +437,9 @@ int nipet_prof_enable(int on);
  * projectors take one image). */
 int nipet_tune_set(int kernel, int width);
 int nipet_tune_get(int kernel, int *width);
-/* Segments per wave run of the back projector at sub-batch width `width` (1, 2
- * or 4): one of the two run lengths compiled for that width (1: 8 or 6;
- * 2: 4 or 6; 4: 6 or 4). Process-wide; set by the autotuner. nipet_tune_get_run
+/* Run-length setting of the back projector at sub-batch width `width` (1, 2 or
+ * 4): 8 or 6; 4 or 6; 6 or 4. Kept and reported; the back projector gives every
+ * wave one run, whatever the setting. nipet_tune_get_run
  * also returns the other compiled length in *alt (may be NULL). No counterpart
  * in the reference (its ray blocks are fixed at compile time). */
 int nipet_tune_set_run(int width, int spw);

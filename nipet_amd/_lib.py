@@ -76,6 +76,8 @@ def lib():
             'nipet_tx_lists': ([P, P, P, P, P], I),
             'nipet_fprj': ([P, P, P, P, I, I, P], I),
             'nipet_fprj_seg': ([P, P, P, P, I, I, P], I),
+            'nipet_bprj_scratch': ([P, I, I], I64),
+            'nipet_scratch_set': ([P, I64], I),
             'nipet_bprj': ([P, P, P, P, I, P], I),
             'nipet_osem_corr': ([P, P, P, P, P, P, I64, P], I),
             'nipet_osem_sens': ([P, P, P, P, I, P], I),
@@ -144,6 +146,32 @@ def ptr(t):
 def stream_handle(device=None):
     import torch
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def bprj_scratch(geom, nprj, nb=1):
+    """Device buffer for staged back projections of ``nprj`` bins of ``nb``
+    images (``nipet_bprj_scratch``), or None where none is used."""
+    import torch
+    n = lib().nipet_bprj_scratch(geom.handle, int(nprj), int(nb))
+    return torch.empty(n, dtype=torch.uint8, device='cuda') if n else None
+
+
+class scratch:
+    """Context manager: this thread's back projections use the device buffer
+    ``buf`` (``nipet_scratch_set``; None: none). The buffer belongs to the
+    stream the calls run on."""
+
+    def __init__(self, buf):
+        self.buf = buf
+
+    def __enter__(self):
+        b = self.buf
+        check(lib().nipet_scratch_set(ptr(b), 0 if b is None else b.numel()),
+              'nipet_scratch_set')
+
+    def __exit__(self, *exc):
+        check(lib().nipet_scratch_set(None, 0), 'nipet_scratch_set')
+        return False
 
 
 class KernelTimer:

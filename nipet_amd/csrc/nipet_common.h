@@ -42,9 +42,13 @@ struct GeomView {
   const float *li_nosi;
   const int16_t *dr_li;
   const uint16_t *sn_mem;
-  const uint16_t *bp_tab;
+  const uint32_t *bp_tab;
+  const uint2 *bp_ev;
+  const uint32_t *bp_off;
+  const int32_t *col_off;
+  const uint32_t *col_ent;
   const int16_t *fp_slot;
-  int naw, nli, ndirect, nsn, dmax, sn_w, fp_nslot;
+  int naw, nli, ndirect, nsn, dmax, sn_w, fp_nslot, maxseg;
   float vox_z;
 };
 
@@ -79,20 +83,46 @@ struct Geom {
   // (d, r0 + k), k < FP_G, of one ring difference; fp_slot[s] = d * 64 + r0
   int16_t *fp_slot = nullptr;
   int fp_nslot = 0;
-  // back-projector LOR tables [3][2][BP_TABN] for 1, 2 and 4 images: byte
-  // offset into the back projector's LDS sinogram row (sinogram * nb * 4) of
-  // LOR (r0, d) and of its mirror at bp_row(d) + d + 1 + r0; the zero row
-  // (nsn * nb * 4) where there is none
-  uint16_t *bp_tab = nullptr;
+  // back-projector LOR table [BP_TN]: at 65 d + r0 the sinograms of LOR (r0, d)
+  // and (<< 16) of its mirror; nsn where there is none
+  uint32_t *bp_tab = nullptr;
+  // z crossings in the order of the back projector's walk (nseg_ev entries, see
+  // bp_event) and the first entry of every segment [nseg + 1]
+  uint2 *bp_ev = nullptr;
+  uint32_t *bp_off = nullptr;
+  // segments by voxel column (CSR): bin << 10 | segment of the bin's list, ascending
+  int32_t *col_off = nullptr;   // [NX * NY + 1]
+  uint32_t *col_ent = nullptr;  // [nseg]
+  int maxseg = 0;               // longest list
   GeomView view = {};           // the pointers above, and
   GeomView *dview = nullptr;    // its copy on the device
 };
 
-// Rows of the back projector's LOR tables: row d holds r0 = -d-1 .. 64
-// (66 + d entries), so that the gather's r0 - h and r0 - e stay in the row.
-constexpr int BP_MAXD = 63;  // largest ring difference of the BP tables
-__host__ __device__ constexpr int bp_row(int d) { return 66 * d + d * (d - 1) / 2; }
-constexpr int BP_TABN = bp_row(BP_MAXD + 1);
+// Rows 0 .. 63 of the back projector's LOR table: row d has its 64 - d LORs at
+// 65 d, then d + 1 zeros up to row d + 1, so that r0 = -d .. 63 reads zeros
+// where there is no LOR; 64 more behind the last row.
+constexpr int BP_MAXD = 63;
+constexpr int BP_TN = 65 * (BP_MAXD + 1) + 64;
+
+// Plane offset of the LORs of one ring difference at t = s (m = 2 d / atn).
+__device__ inline int plane_offset(double m, double s) { return (int)floor(fma(m, s, 0.5)); }
+
+// Entry of Geom::bp_ev: the LORs of ring difference d pass from plane offset w
+// to w + 1, beta before the segment's end. A float64 +beta (w even) or -beta
+// (odd) with its low 23 bits (2^-30 of beta) replaced by: 1 for the segment's
+// last entry, 4 D, and d << 16. The LORs are at entries D + i, D + i + 1 (one
+// direction, planes 2 i and 2 i + 1) and BP_TN + 1 + 129 d - D + i (the other,
+// both planes) of the kernel's table: vb, one unused entry, va. A segment
+// without crossings has one entry of ring difference 64, which has no LORs.
+__host__ __device__ constexpr uint32_t bp_entry(int d, int w) {
+  return w & 1 ? BP_TN + 65 * d - (w >> 1) : 64 * d + (w >> 1);
+}
+__device__ inline uint2 bp_event(int d, int w, double beta, bool last) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(w & 1 ? -beta : beta);
+  return make_uint2(((uint32_t)b & 0xff800000u) | (uint32_t)d << 16 | bp_entry(d, w) << 2 |
+                        (last ? 1u : 0u),
+                    (uint32_t)(b >> 32));
+}
 
 // Position of plane w in the forward projector's LDS rows (64 even planes, then
 // 64 odd ones, of 8 bytes), in bytes.

@@ -269,6 +269,67 @@ __global__ __launch_bounds__(256) void k_events(const int32_t *__restrict__ off,
   }
 }
 
+// Geom::bp_ev of one bin per wave, lane d its ring difference d: the number of
+// entries (ev NULL), or the entries from base[bin] on and the segments' offsets.
+__global__ __launch_bounds__(64) void k_bp_events(const int32_t *__restrict__ off,
+                                                  const SegRec *__restrict__ seg,
+                                                  const double *__restrict__ atn, int dmax,
+                                                  uint32_t *__restrict__ base,
+                                                  uint2 *__restrict__ ev,
+                                                  uint32_t *__restrict__ ev_off) {
+  const int aw = blockIdx.x, lane = threadIdx.x, beg = off[aw], n = off[aw + 1] - beg;
+  const bool on = lane >= 1 && lane <= dmax;
+  const double at = atn[aw], m = on ? 2.0 * lane / at : 0.0, inv = on ? at / (2.0 * lane) : 0.0;
+  const unsigned long long below = (1ull << lane) - 1;
+  uint32_t pos = ev ? base[aw] : 0;
+  int w = n > 0 ? plane_offset(m, seg[beg].s) : 0;
+  for (int j = 0; j < n; j++) {
+    const double s = seg[beg + j].s,
+                 s1 = j + 1 < n ? seg[beg + j + 1].s : s + (double)seg[beg + j].len;
+    const int wn = plane_offset(m, s1);
+    if (ev && lane == 0) ev_off[beg + j] = pos;
+    if (!__any(w < wn)) {
+      if (ev && lane == 0) ev[pos] = bp_event(BP_MAXD + 1, 0, 0.0, true);
+      pos++;
+    }
+    for (unsigned long long hit; (hit = __ballot(w < wn)) != 0;) {
+      const bool last = !__any(w + 1 < wn);
+      if (ev && w < wn) {
+        const double beta = fmin(fmax(s1 - ((double)w + 0.5) * inv, 0.0), s1 - s);
+        ev[pos + __popcll(hit & below)] = bp_event(lane, w, beta, last && !(hit >> lane >> 1));
+      }
+      pos += __popcll(hit);
+      w += w < wn ? 1 : 0;
+    }
+  }
+  if (!ev && lane == 0) base[aw] = pos;
+}
+
+// Segments by voxel column (Geom::col_off, col_ent): counts per column, then
+// entries in any order, then each column's entries in ascending order (the rank
+// of every entry among the column's, n^2 comparisons of a few hundred).
+__global__ void k_col_count(const SegRec *__restrict__ seg, int64_t n, int32_t *cnt) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) atomicAdd(cnt + seg[i].colz / NZ, 1);
+}
+__global__ void k_col_fill(const int32_t *__restrict__ off, const SegRec *__restrict__ seg,
+                           int naw, int32_t *cur, uint32_t *ent) {
+  const int aw = blockIdx.x;
+  for (int k = off[aw] + threadIdx.x; k < off[aw + 1]; k += blockDim.x)
+    ent[atomicAdd(cur + seg[k].colz / NZ, 1)] = (uint32_t)aw << 10 | (uint32_t)(k - off[aw]);
+}
+__global__ __launch_bounds__(64) void k_col_sort(const int32_t *__restrict__ col_off,
+                                                 const uint32_t *__restrict__ in,
+                                                 uint32_t *__restrict__ out) {
+  const int b = col_off[blockIdx.x], n = col_off[blockIdx.x + 1] - b;
+  for (int i = threadIdx.x; i < n; i += 64) {
+    const uint32_t e = in[b + i];
+    int rank = 0;
+    for (int j = 0; j < n; j++) rank += in[b + j] < e ? 1 : 0;
+    out[b + rank] = e;
+  }
+}
+
 // Bins of a subset ordered by decreasing segment count (bins outside
 // 0 .. naw-1 last), one workgroup: a counting sort by count with LDS buckets.
 // Bins of equal count keep no particular order: the order only decides which
@@ -345,7 +406,9 @@ int nipet_prof_read(int kernel, double *total_ms, int64_t *count) {
 static void geom_free(Geom *g) {
   // teardown: a failing free leaves nothing to undo
   void *bufs[] = {g->off,   g->seg,    g->atn,    g->lmax,   g->li_z,   g->li_sn,
-                  g->li_nosi, g->dr_li, g->sn_mem, g->fp_slot, g->bp_tab, g->ev, g->dview};
+                  g->li_nosi, g->dr_li, g->sn_mem, g->fp_slot, g->bp_tab, g->bp_ev,
+                  g->bp_off, g->ev, g->dview,
+                  g->col_off, g->col_ent};
   for (void *p : bufs) (void)hipFree(p);
 }
 
@@ -449,28 +512,18 @@ static int geom_build(const NipetGeomDesc *d, NipetGeom *g) {
     NIPET_HIP(hipMemcpy(g->fp_slot, slots.data(), slots.size() * sizeof(int16_t),
                         hipMemcpyHostToDevice));
   }
+  if (d->nsn > 4095) {
+    set_error("%d sinograms: at most 4095", d->nsn);
+    return NIPET_EINVAL;
+  }
   {
-    // back-projector LOR tables, scaled for 1, 2 and 4 images: 16-bit byte
-    // offsets into a row of nsn + 1 sinograms of 4 images
-    if (d->nsn * 4 * 4 > 0xffff) {
-      set_error("%d sinograms: the back projector's 16-bit row offsets reach 4095", d->nsn);
-      return NIPET_EINVAL;
+    std::vector<uint32_t> tab(BP_TN, (uint32_t)d->nsn * 0x10001u);
+    for (int li = 0; li < d->nli; li++) {
+      const int r0 = (int)floorf(liz[li].x) >> 1, dd = (int)liz[li].y >> 1;
+      tab[65 * dd + r0] = (uint32_t)lisn[li].x | (uint32_t)(dd > 0 ? lisn[li].y : d->nsn) << 16;
     }
-    std::vector<uint16_t> tab(6 * (size_t)BP_TABN);
-    const int nbs[3] = {1, 2, 4};
-    for (int w = 0; w < 3; w++) {
-      uint16_t *t = tab.data() + (size_t)w * 2 * BP_TABN;
-      const uint16_t zr = (uint16_t)(d->nsn * nbs[w] * 4);
-      for (int i = 0; i < 2 * BP_TABN; i++) t[i] = zr;
-      for (int li = 0; li < d->nli; li++) {
-        const int r0 = (int)floorf(liz[li].x) >> 1, dd = (int)liz[li].y >> 1;
-        const int k = bp_row(dd) + dd + 1 + r0;
-        t[k] = (uint16_t)(lisn[li].x * nbs[w] * 4);
-        if (dd > 0) t[BP_TABN + k] = (uint16_t)(lisn[li].y * nbs[w] * 4);
-      }
-    }
-    NIPET_HIP(hipMalloc(&g->bp_tab, tab.size() * sizeof(uint16_t)));
-    NIPET_HIP(hipMemcpy(g->bp_tab, tab.data(), tab.size() * sizeof(uint16_t),
+    NIPET_HIP(hipMalloc(&g->bp_tab, tab.size() * sizeof(uint32_t)));
+    NIPET_HIP(hipMemcpy(g->bp_tab, tab.data(), tab.size() * sizeof(uint32_t),
                         hipMemcpyHostToDevice));
   }
   NIPET_HIP(hipMalloc(&g->dr_li, drli.size() * sizeof(int16_t)));
@@ -566,6 +619,65 @@ static int geom_build(const NipetGeomDesc *d, NipetGeom *g) {
         return NIPET_EINVAL;
       }
   }
+  {
+    uint32_t *base = nullptr;
+    struct Tmp3 {
+      uint32_t **p;
+      ~Tmp3() { (void)hipFree(*p); }
+    } tmp3{&base};
+    NIPET_HIP(hipMalloc(&base, d->naw * sizeof(uint32_t)));
+    k_bp_events<<<d->naw, 64>>>(g->off, g->seg, g->atn, g->dmax, base, nullptr, nullptr);
+    NIPET_HIP(hipGetLastError());
+    std::vector<uint32_t> be(d->naw);
+    NIPET_HIP(hipMemcpy(be.data(), base, d->naw * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    uint64_t ne = 0;
+    for (uint32_t &b : be) {
+      const uint32_t c = b;
+      b = (uint32_t)ne;
+      ne += c;
+    }
+    if (ne > UINT32_MAX) {
+      set_error("too many z crossings");
+      return NIPET_EINVAL;
+    }
+    const uint32_t end = (uint32_t)ne;
+    // (entries are read in eights, one eight ahead)
+    NIPET_HIP(hipMalloc(&g->bp_ev, (ne + 24) * sizeof(uint2)));
+    NIPET_HIP(hipMemset(g->bp_ev + ne, 0, 24 * sizeof(uint2)));
+    NIPET_HIP(hipMalloc(&g->bp_off, (tot + 1) * sizeof(uint32_t)));
+    NIPET_HIP(hipMemcpy(g->bp_off + tot, &end, sizeof(end), hipMemcpyHostToDevice));
+    NIPET_HIP(hipMemcpy(base, be.data(), d->naw * sizeof(uint32_t), hipMemcpyHostToDevice));
+    k_bp_events<<<d->naw, 64>>>(g->off, g->seg, g->atn, g->dmax, base, g->bp_ev, g->bp_off);
+    NIPET_HIP(hipGetLastError());
+    NIPET_HIP(hipDeviceSynchronize());
+  }
+  {
+    for (int i = 0; i < d->naw; i++) g->maxseg = std::max(g->maxseg, (int)cnt[i]);
+    int32_t *cur = nullptr;
+    uint32_t *ent = nullptr;
+    struct Tmp2 {
+      void **p[2];
+      ~Tmp2() {
+        for (void **q : p) (void)hipFree(*q);
+      }
+    } tmp2{{(void **)&cur, (void **)&ent}};
+    const size_t nc = NX * NY;
+    NIPET_HIP(hipMalloc(&cur, nc * sizeof(int32_t)));
+    NIPET_HIP(hipMalloc(&ent, (tot + 1) * sizeof(uint32_t)));
+    NIPET_HIP(hipMalloc(&g->col_off, (nc + 1) * sizeof(int32_t)));
+    NIPET_HIP(hipMalloc(&g->col_ent, (tot + 1) * sizeof(uint32_t)));
+    NIPET_HIP(hipMemset(cur, 0, nc * sizeof(int32_t)));
+    if (tot > 0) k_col_count<<<(unsigned)((tot + 255) / 256), 256>>>(g->seg, tot, cur);
+    std::vector<int32_t> co(nc + 1, 0);
+    NIPET_HIP(hipMemcpy(co.data() + 1, cur, nc * sizeof(int32_t), hipMemcpyDeviceToHost));
+    for (size_t i = 0; i < nc; i++) co[i + 1] += co[i];
+    NIPET_HIP(hipMemcpy(g->col_off, co.data(), (nc + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
+    NIPET_HIP(hipMemcpy(cur, co.data(), nc * sizeof(int32_t), hipMemcpyHostToDevice));
+    k_col_fill<<<d->naw, 256>>>(g->off, g->seg, d->naw, cur, ent);
+    k_col_sort<<<(unsigned)nc, 64>>>(g->col_off, ent, g->col_ent);
+    NIPET_HIP(hipGetLastError());
+    NIPET_HIP(hipDeviceSynchronize());
+  }
   GeomView &v = g->view;
   v.off = g->off;
   v.seg = g->seg;
@@ -578,6 +690,11 @@ static int geom_build(const NipetGeomDesc *d, NipetGeom *g) {
   v.dr_li = g->dr_li;
   v.sn_mem = g->sn_mem;
   v.bp_tab = g->bp_tab;
+  v.bp_ev = g->bp_ev;
+  v.bp_off = g->bp_off;
+  v.col_off = g->col_off;
+  v.col_ent = g->col_ent;
+  v.maxseg = g->maxseg;
   v.fp_slot = g->fp_slot;
   v.fp_nslot = g->fp_nslot;
   v.naw = g->naw;

@@ -77,9 +77,10 @@ class Projector:
         torch = _torch()
         g = self.geom if geom is None else geom
         out = torch.empty((320, 320, 127), dtype=torch.float32, device=sino.device)
-        _lib.check(_lib.lib().nipet_bprj(g.handle, _lib.ptr(out), _lib.ptr(sino),
-                                         _lib.ptr(self.subs), self.nprj, _lib.stream_handle()),
-                   'nipet_bprj')
+        with _lib.scratch(_lib.bprj_scratch(g, self.nprj)):
+            _lib.check(_lib.lib().nipet_bprj(g.handle, _lib.ptr(out), _lib.ptr(sino),
+                                             _lib.ptr(self.subs), self.nprj,
+                                             _lib.stream_handle()), 'nipet_bprj')
         return out
 
     def span1(self):

@@ -91,9 +91,11 @@ def autotune(state, widths=(4, 2, 1), repeats=2, probe=4):
                                                  _lib.ptr(subs), nprj, n, 0, st), 'nipet_fprj_b')
 
     def bprj(n):
-        return lambda: _lib.check(L.nipet_bprj_b(state.geom.handle, _lib.ptr(bimg),
-                                                 _lib.ptr(sino), _lib.ptr(subs), nprj, n, st),
-                                  'nipet_bprj_b')
+        def launch():
+            with _lib.scratch(state.scratch):
+                _lib.check(L.nipet_bprj_b(state.geom.handle, _lib.ptr(bimg), _lib.ptr(sino),
+                                          _lib.ptr(subs), nprj, n, st), 'nipet_bprj_b')
+        return launch
     best = None
     for w in widths:
         n = min(w, nb)
@@ -143,7 +145,8 @@ def prepare_groups(scanner_params, prompt_groups, asng, nsng, rsng=None, ssng=No
     per = _per_rep(rsng) or _per_rep(ssng)
     for p in prompt_groups:
         g = p.shape[2]
-        work = None if first is None else (first.work_sino, first.work_img, first.work_img2)
+        work = None if first is None else (first.work_sino, first.work_img, first.work_img2,
+                                          first.scratch)
         if first is not None and not per:
             st = OsemBatch(first.geom, first.subsets, p, first.rho, False, first.sens,
                            first.mask, g, work=work, krnl=first.krnl, win=first.win)
@@ -396,7 +399,8 @@ def replicates_and_frames(words, scanner_params, asng, nsng, rs, nrep=64, seed=1
         frm.append(osem_prepare_batch(scanner_params, p, asng, nsng,
                                       frho[..., off:off + g].contiguous(), None,
                                       sens=first.sens, psf=psf,
-                                      work=(first.work_sino, first.work_img, first.work_img2)))
+                                      work=(first.work_sino, first.work_img, first.work_img2,
+                                            first.scratch)))
         off += g
     del frho
     mark('prepare_s')

@@ -158,8 +158,10 @@ def back_prj(sino, scanner_params, isub=ISUB_DEFAULT, dev_out=False, output=None
         bimg, _ = _dev_tensor(output, torch.float32)
         if tuple(bimg.shape) != shape:
             raise ValueError(f'output must have shape {shape}')
-    _lib.check(_lib.lib().nipet_bprj(geom.handle, _lib.ptr(bimg), _lib.ptr(sinog), _lib.ptr(subs),
-                                     nprj, _lib.stream_handle()), 'nipet_bprj')
+    with _lib.scratch(_lib.bprj_scratch(geom, nprj)):
+        _lib.check(_lib.lib().nipet_bprj(geom.handle, _lib.ptr(bimg), _lib.ptr(sinog),
+                                         _lib.ptr(subs), nprj, _lib.stream_handle()),
+                   'nipet_bprj')
     if not dev_out:
         from ..img.mmrimg import convert2e7
         _sync(True)

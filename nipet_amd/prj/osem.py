@@ -145,6 +145,8 @@ class OsemState:
         self.krnl = krnl
         self.work_img2 = None if krnl is None else torch.empty_like(self.work_img)
         self._pair = None
+        # staged back projections (two images while sensitivities are pending)
+        self.scratch = _lib.bprj_scratch(geom, self.nprj, 2 if self.pending else 1)
 
     @property
     def sens(self):
@@ -153,7 +155,8 @@ class OsemState:
         mask's segment windows: it is exact on the mask, which is all the
         update reads.)"""
         for k in sorted(self.pending):
-            sensitivity(self.geom, self.an, self.subsets[k], out=self._sens[k])
+            sensitivity(self.geom, self.an, self.subsets[k], out=self._sens[k],
+                        scratch=self.scratch)
         self.pending.clear()
         return self._sens
 
@@ -168,15 +171,17 @@ class OsemState:
         return self._pair
 
 
-def sensitivity(geom, an, subs, out=None):
+def sensitivity(geom, an, subs, out=None, scratch=None):
     """BP_subset(a*n) (``prj/mmrrec.py:291-298``) for one subset (device tensors:
-    ``an`` the full (Naw, nsn) a*n sinogram, read at the subset's bins)."""
+    ``an`` the full (Naw, nsn) a*n sinogram, read at the subset's bins;
+    ``scratch``: the back projection's buffer, made when None)."""
     torch = _torch()
     if out is None:
         out = torch.empty((320, 320, 127), dtype=torch.float32, device='cuda')
-    _lib.check(_lib.lib().nipet_osem_sens(geom.handle, _lib.ptr(out), _lib.ptr(an),
-                                          _lib.ptr(subs), len(subs), _lib.stream_handle()),
-               'nipet_osem_sens')
+    with _lib.scratch(_lib.bprj_scratch(geom, len(subs)) if scratch is None else scratch):
+        _lib.check(_lib.lib().nipet_osem_sens(geom.handle, _lib.ptr(out), _lib.ptr(an),
+                                              _lib.ptr(subs), len(subs), _lib.stream_handle()),
+                   'nipet_osem_sens')
     return out
 
 
@@ -268,6 +273,11 @@ def osem_iteration(state, img, first_full=True):
     Every update after the first walks the mask's segment windows (the image
     is then zero outside the mask); the first does too when ``first_full`` is
     False (an image already masked by an earlier update)."""
+    with _lib.scratch(state.scratch):
+        _subsets(state, img, first_full)
+
+
+def _subsets(state, img, first_full):
     st = _lib.stream_handle()
     L = _lib.lib()
     for k, subs in enumerate(state.subsets):
@@ -329,7 +339,7 @@ class OsemBatch:
         self.prompts, self.rho, self.rho_per_rep, self.sens, self.mask = (
             prompts, rho, rho_per_rep, sens, mask)
         self.nprj = max(len(s) for s in subsets)
-        if work is not None:  # (work_sino, work_img[, work_img2]) of another batch
+        if work is not None:  # (work_sino, work_img[, work_img2[, scratch]]) of another batch
             ws, wi = work[0], work[1]
             if ws.numel() < self.nprj * geom.nsn * nb or wi.numel() < NVOX * nb:
                 raise ValueError('shared work buffers are too small for this batch')
@@ -339,6 +349,11 @@ class OsemBatch:
                                          device='cuda')
             self.work_img = torch.empty((320, 320, 127, nb), dtype=torch.float32,
                                         device='cuda')
+        # staged back projections (shared like the other buffers)
+        need = _lib.lib().nipet_bprj_scratch(geom.handle, self.nprj, nb)
+        old = work[3] if work is not None and len(work) > 3 else None
+        self.scratch = old if old is not None and old.numel() >= need else \
+            _lib.bprj_scratch(geom, self.nprj, nb)
         self.work_img2 = None
         if krnl is not None:  # resolution modelling: a second work image
             self.work_img2 = (work[2] if work is not None and len(work) > 2 and
@@ -409,6 +424,11 @@ def osem_prepare_batch(scanner_params, prompts, asng, nsng, rsng=None, ssng=None
 
 def osem_iteration_batch(state, img, first_full=True):
     """One OSEM iteration of all nb images; windows as ``osem_iteration``."""
+    with _lib.scratch(state.scratch):
+        _subsets_batch(state, img, first_full)
+
+
+def _subsets_batch(state, img, first_full):
     st = _lib.stream_handle()
     L = _lib.lib()
     for k, subs in enumerate(state.subsets):

@@ -95,8 +95,9 @@ def bprj(bimg, sino, txLUT, axLUT, subs, cnst, sync=True):
     y, _ = _dev(sino, torch.float32)
     if y.numel() != nprj * g.nsn or out.numel() != 320 * 320 * 127:
         raise ValueError(f'bprj: sino must hold ({nprj}, {g.nsn}) values and bimg 320*320*127')
-    _lib.check(_lib.lib().nipet_bprj(g.handle, _lib.ptr(out), _lib.ptr(y), _lib.ptr(rows), nprj,
-                                     _lib.stream_handle()), 'nipet_bprj')
+    with _lib.scratch(_lib.bprj_scratch(g, nprj)):
+        _lib.check(_lib.lib().nipet_bprj(g.handle, _lib.ptr(out), _lib.ptr(y), _lib.ptr(rows),
+                                         nprj, _lib.stream_handle()), 'nipet_bprj')
     _done(out, host, sync)
 
 
@@ -152,8 +153,9 @@ def osem(imgout, psng, rsng, ssng, nsng, asng, subs, imgsens, rcnmsk, krnl, txLU
         k = np.ascontiguousarray(np.asarray(krnl, np.float32))
         if k.shape != (3, 17):
             raise ValueError('krnl must be (3, 17)')
-    _lib.check(_lib.lib().nipet_osem_iter(
-        g.handle, _lib.ptr(img), _lib.ptr(p), _lib.ptr(r), _lib.ptr(s), _lib.ptr(n), _lib.ptr(a),
-        table.ctypes.data, nsub, stride, _lib.ptr(sens), _lib.ptr(m),
-        None if k is None else k.ctypes.data, _lib.stream_handle()), 'nipet_osem_iter')
+    with _lib.scratch(_lib.bprj_scratch(g, max(stride - 1, 0))):
+        _lib.check(_lib.lib().nipet_osem_iter(
+            g.handle, _lib.ptr(img), _lib.ptr(p), _lib.ptr(r), _lib.ptr(s), _lib.ptr(n),
+            _lib.ptr(a), table.ctypes.data, nsub, stride, _lib.ptr(sens), _lib.ptr(m),
+            None if k is None else k.ctypes.data, _lib.stream_handle()), 'nipet_osem_iter')
     _done(img, host)

@@ -164,3 +164,84 @@ def test_window_is_the_masked_image(torch, lib, params, span):
         outs.append(work)
     close(torch, outs[1], outs[0])
     assert isinstance(geom.handle, ct.c_void_p)
+
+
+# ------------------------------------------------------------ back projection
+def back(torch, lib, geom, sino, rows, scratch_rows=None, nb=1):
+    """``nipet_bprj_b`` without scratch (atomics), or staged with room for
+    ``scratch_rows`` bins a pass."""
+    img = torch.full((320, 320, 127) + ((nb,) if nb > 1 else ()), 3.0, device='cuda')
+    buf = None
+    if scratch_rows:
+        full = lib.lib().nipet_bprj_scratch(geom.handle, len(rows), nb)
+        one = lib.lib().nipet_bprj_scratch(geom.handle, 2001, nb) - \
+            lib.lib().nipet_bprj_scratch(geom.handle, 2000, nb)
+        n = full - (len(rows) - min(scratch_rows, len(rows))) * one
+        buf = torch.full((n,), 255, dtype=torch.uint8, device='cuda')
+    with lib.scratch(buf):
+        lib.check(lib.lib().nipet_bprj_b(geom.handle, lib.ptr(img), lib.ptr(sino), lib.ptr(rows),
+                                         len(rows), nb, lib.stream_handle()), 'nipet_bprj_b')
+    return img
+
+
+def exact_back(torch, params, sino, rows):
+    from oracle import oracle as O
+    return torch.from_numpy(O.bprj(params, sino.cpu().numpy(), rows.cpu().numpy())).cuda()
+
+
+@pytest.mark.parametrize('kind', ['signed', 'one bin', 'huge beside small'])
+def test_back_projection_sums_return_to_zero(torch, lib, params, kind):
+    """The plane sums along a ray hold what enters and leaves: voxels that no
+    LOR with a value touches get exactly 0, and small values beside huge ones
+    keep their precision (a sum of a voxel's own terms bounds its error)."""
+    from nipet_amd.geom import get_geom
+    geom, rows = get_geom(params), rows_of(torch, 1 if kind == 'one bin' else 23, 21)
+    g = torch.Generator(device='cuda').manual_seed(2)
+    y = torch.rand((len(rows), geom.nsn), generator=g, device='cuda')
+    y = y * (torch.rand(y.shape, generator=g, device='cuda') < 0.05)
+    if kind == 'signed':
+        y = y * torch.sign(torch.rand(y.shape, generator=g, device='cuda') - 0.5)
+    elif kind != 'one bin':
+        y[:, ::3] *= 1e6
+    got = back(torch, lib, geom, y, rows).double()
+    ref, top = exact_back(torch, params, y, rows), exact_back(torch, params, y.abs(), rows)
+    assert bool((got[top == 0] == 0).all())
+    assert float(((got - ref).abs() / top.clamp(min=1e-3 if kind != 'one bin' else 1e-4)).max()) < BAR
+
+
+@pytest.mark.parametrize('bad', [float('inf'), float('nan')])
+def test_back_projection_non_finite(torch, lib, params, bad):
+    """A non-finite sinogram value reaches the voxels of its LORs and no others."""
+    from nipet_amd.geom import get_geom
+    geom, rows = get_geom(params), rows_of(torch, 9, 22)
+    y = torch.rand((len(rows), geom.nsn), device='cuda')
+    one = torch.zeros_like(y)
+    one[4, 400] = 1.0
+    hit = exact_back(torch, params, one, rows) > 0
+    clean = y.clone()
+    clean[4, 400] = 0.0
+    y[4, 400] = bad
+    got = back(torch, lib, geom, y, rows)
+    assert not bool(torch.isfinite(got[hit]).any())
+    close(torch, got[~hit], exact_back(torch, params, clean, rows)[~hit])
+
+
+@pytest.mark.parametrize('nb', [1, 2, 3])
+@pytest.mark.parametrize('n,per', [(1536, 1536), (1700, 1537), (3400, 1600)])
+def test_staged_equals_atomics(torch, lib, params, n, per, nb):
+    """Staged rows gathered in one or several passes against float atomics:
+    duplicated and invalid bins, odd batches, twice the same bits."""
+    from nipet_amd.geom import get_geom
+    geom, rows = get_geom(params), rows_of(torch, n, 23)
+    rows[7], rows[n // 2], rows[n - 1] = rows[11], -1, 68516
+    g = torch.Generator(device='cuda').manual_seed(4)
+    y = torch.rand((n, geom.nsn) + ((nb,) if nb > 1 else ()), generator=g, device='cuda')
+    ref = back(torch, lib, geom, y, rows, None, nb).double()
+    got = back(torch, lib, geom, y, rows, per, nb)
+    assert torch.equal(got, back(torch, lib, geom, y, rows, per, nb))
+    assert float((got - ref).abs().max()) < BAR * float(ref.max())
+    assert torch.equal(got == 0, ref == 0)
+    if nb > 1:
+        for b in range(nb):
+            one = back(torch, lib, geom, y[..., b].contiguous(), rows, n)
+            assert float((got[..., b] - one).abs().max()) < 1e-6 * float(one.max())
