@@ -314,6 +314,17 @@ typedef struct {
 } NipetLmOut;
 
 int nipet_lm_create(const NipetLmConfig *cfg, NipetLm **out);
+/* nipet_lm_create / nipet_lm_chunk in the caller's device memory (aligned to 256
+ * bytes; the session's until it is destroyed and its kernels have run, a chunk's
+ * until the chunk's kernels have run; NULL: allocated by the call). A session
+ * of 600 M words allocates and frees 4.9 GB otherwise, which took 130 of 143 ms.
+ * nipet_lm_bytes / nipet_lm_work_bytes: the sizes (0: invalid argument). */
+int64_t nipet_lm_bytes(const NipetLmConfig *cfg);
+int nipet_lm_create_in(const NipetLmConfig *cfg, void *mem, int64_t bytes, void *stream,
+                       NipetLm **out);
+int64_t nipet_lm_work_bytes(const NipetLm *h, int64_t n);
+int nipet_lm_chunk_in(NipetLm *h, const int32_t *words, int64_t n, const NipetLmOut *out,
+                      void *work, int64_t bytes, void *stream);
 /* Histogram words[0..n) (device int32) on `stream`. A chunk that fails after
  * its first kernels were queued (a device allocation for the staging slots)
  * leaves the session unusable: later chunk / finish calls return an error. */

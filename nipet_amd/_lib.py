@@ -101,6 +101,10 @@ def lib():
             'nipet_osem_subset_b': ([P, P, P, P, I, P, I, P, P, P, I, I, P, P, P], I),
             'nipet_lm_create': ([ct.POINTER(NipetLmConfig), ct.POINTER(P)], I),
             'nipet_lm_chunk': ([P, P, I64, ct.POINTER(NipetLmOut), P], I),
+            'nipet_lm_bytes': ([ct.POINTER(NipetLmConfig)], I64),
+            'nipet_lm_create_in': ([ct.POINTER(NipetLmConfig), P, I64, P, ct.POINTER(P)], I),
+            'nipet_lm_work_bytes': ([P, I64], I64),
+            'nipet_lm_chunk_in': ([P, P, I64, ct.POINTER(NipetLmOut), P, I64, P], I),
             'nipet_lm_status': ([P, P, P, P], I),
             'nipet_lm_finish': ([P, ct.POINTER(NipetLmOut), P], I),
             'nipet_lm_destroy': ([P], None),

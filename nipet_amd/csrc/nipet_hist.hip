@@ -31,6 +31,7 @@
 //  k_lm_sgl_first / k_lm_sgl_apply  singles buckets in two order-free passes.
 #include <stdlib.h>
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -1079,7 +1080,8 @@ struct NipetLm {
   unsigned long long *sgl_idx = nullptr;
   int32_t *sgl_word = nullptr, *sgl_ms = nullptr;
   unsigned int *sgl_count = nullptr, *bad = nullptr;
-  unsigned int sgl_cap = 0;
+  unsigned int sgl_cap = 0;   // entries of the session's own list
+  unsigned int sgl_used = 0;  // the last chunk's capacity
   int32_t *ssrb_off = nullptr, *ssrb_list = nullptr;  // sinograms of each SSRB plane
   int64_t base = 0;  // global index of the next word
   // LDS-privatised sinogram counts: buckets of LM_BBINS output bins (nbk),
@@ -1094,14 +1096,59 @@ struct NipetLm {
   // set when a chunk failed after its first kernels had advanced the
   // session's time-tag carry: the session can no longer be continued
   bool broken = false;
+  void *own = nullptr;  // the session's memory, or NULL where it is the caller's
 };
 
 static void lm_free(NipetLm *h) {
-  void *ps[] = {h->lut, h->rno, h->s2cF, h->cdf, h->carry, h->blk_last, h->blk_carry,
-                h->first_nz, h->sgl_idx, h->sgl_word, h->sgl_ms, h->sgl_count, h->bad,
-                h->ssrb_off, h->ssrb_list, h->gcnt, h->bstart, h->bcur, h->gccnt,
-                h->cstart, h->ccur, h->stage, h->stage2, h->fan_part};
+  void *ps[] = {h->blk_last, h->blk_carry, h->sgl_idx, h->sgl_word, h->sgl_ms, h->stage,
+                h->stage2, h->own};
   for (void *q : ps) (void)hipFree(q);
+}
+
+// Arrays laid out one behind the other, each aligned to 256 bytes. With base
+// NULL only their size is counted.
+struct LmLayout {
+  char *base;
+  int64_t bytes = 0;
+  template <typename T>
+  T *take(int64_t n) {
+    T *p = base ? (T *)(base + bytes) : nullptr;
+    bytes += (std::max<int64_t>(n, 1) * (int64_t)sizeof(T) + 255) / 256 * 256;
+    return p;
+  }
+};
+
+static int lm_nsino(const NipetLmConfig *c) {
+  return c->span == 11 ? 837 : (c->span == 1 ? NSN1 : SEG0);
+}
+
+// The session's arrays: tables written by the host first (their bytes are
+// returned), then what kernels fill.
+static int64_t lm_layout(const NipetLmConfig *c, NipetLm *h, LmLayout &l) {
+  h->nbins = (int64_t)lm_nsino(c) * NSBINANG;
+  h->nbk = (int)((h->nbins + LM_BBINS - 1) >> LM_BSHIFT);
+  h->ncb = (int)((h->nbins + (1 << LM_CSHIFT) - 1) >> LM_CSHIFT);
+  h->ssrb_off = l.take<int32_t>(SEG0 + 1);
+  h->ssrb_list = l.take<int32_t>(lm_nsino(c));
+  h->lut = l.take<int32_t>(NSN1);
+  h->rno = l.take<short2>(NSN1);
+  h->s2cF = l.take<short2>(NSBINANG);
+  h->cdf = l.take<uint32_t>(LM_NCDF);
+  h->carry = l.take<int32_t>(1);
+  h->bad = l.take<unsigned int>(1);
+  h->sgl_count = l.take<unsigned int>(1);
+  const int64_t tables = l.bytes;
+  h->first_nz = l.take<unsigned long long>((int64_t)c->nitag * NBUCKTS);
+  if (c->nrep == 1 && c->btp != 1) {  // LDS-privatised sinogram counts
+    h->gcnt = l.take<uint32_t>(h->nbk);
+    h->bstart = l.take<uint32_t>(h->nbk + 1);
+    h->bcur = l.take<uint32_t>(h->nbk);
+    h->gccnt = l.take<uint32_t>(h->ncb);
+    h->cstart = l.take<uint32_t>(h->ncb + 1);
+    h->ccur = l.take<uint32_t>(h->ncb);
+    h->fan_part = l.take<uint32_t>((int64_t)LM_FAN_WG * LM_FAN);
+  }
+  return tables;
 }
 
 // uint32 Poisson CDF (same formula and order as the CPU definition)
@@ -1115,7 +1162,8 @@ static void poisson_cdf(double lambda, uint32_t *cdf, int K) {
   }
 }
 
-static int lm_build(const NipetLmConfig *c, NipetLm *h) {
+// Builds the session in mem (lm_layout's bytes on the current device).
+static int lm_build(const NipetLmConfig *c, NipetLm *h, void *mem, hipStream_t st) {
   NIPET_HIP(hipGetDevice(&h->device));
   std::vector<int32_t> lut(NSN1);
   for (int i = 0; i < NSN1; i++) {
@@ -1138,7 +1186,7 @@ static int lm_build(const NipetLmConfig *c, NipetLm *h) {
   uint32_t cdf[LM_NCDF];
   poisson_cdf(c->btprt, cdf, LM_NCDF);
   // sinograms of the output span that fall on each SSRB plane
-  const int nsino = c->span == 11 ? 837 : (c->span == 1 ? NSN1 : SEG0);
+  const int nsino = lm_nsino(c);
   std::vector<int> plane_of(nsino, -1);
   for (int si = 0; si < NSN1; si++) {
     int s = c->span == 11 ? c->sn1_sn11[si] : (c->span == 1 ? si : c->sn1_ssrb[si]);
@@ -1158,44 +1206,27 @@ static int lm_build(const NipetLmConfig *c, NipetLm *h) {
       if (plane_of[s] == pl) slist.push_back(s);
     soff[pl + 1] = (int32_t)slist.size();
   }
-  NIPET_HIP(hipMalloc(&h->ssrb_off, (SEG0 + 1) * sizeof(int32_t)));
-  NIPET_HIP(hipMalloc(&h->ssrb_list, std::max<size_t>(slist.size(), 1) * sizeof(int32_t)));
-  NIPET_HIP(hipMemcpy(h->ssrb_off, soff.data(), (SEG0 + 1) * sizeof(int32_t),
-                      hipMemcpyHostToDevice));
-  if (!slist.empty())
-    NIPET_HIP(hipMemcpy(h->ssrb_list, slist.data(), slist.size() * sizeof(int32_t),
-                        hipMemcpyHostToDevice));
-  NIPET_HIP(hipMalloc(&h->lut, NSN1 * sizeof(int32_t)));
-  NIPET_HIP(hipMalloc(&h->rno, NSN1 * sizeof(short2)));
-  NIPET_HIP(hipMalloc(&h->s2cF, NSBINANG * sizeof(short2)));
-  NIPET_HIP(hipMalloc(&h->cdf, LM_NCDF * sizeof(uint32_t)));
-  NIPET_HIP(hipMalloc(&h->carry, sizeof(int32_t)));
-  NIPET_HIP(hipMalloc(&h->sgl_count, sizeof(unsigned int)));
-  NIPET_HIP(hipMalloc(&h->bad, sizeof(unsigned int)));
-  NIPET_HIP(hipMalloc(&h->first_nz, (size_t)c->nitag * NBUCKTS * sizeof(unsigned long long)));
-  h->nbins = (int64_t)nsino * NSBINANG;
-  h->nbk = (int)((h->nbins + LM_BBINS - 1) >> LM_BSHIFT);
-  h->ncb = (int)((h->nbins + (1 << LM_CSHIFT) - 1) >> LM_CSHIFT);
-  if (c->nrep == 1 && c->btp != 1) {  // LDS-privatised sinogram counts
-    NIPET_HIP(hipMalloc(&h->gcnt, (size_t)h->nbk * sizeof(uint32_t)));
-    NIPET_HIP(hipMalloc(&h->bstart, (size_t)(h->nbk + 1) * sizeof(uint32_t)));
-    NIPET_HIP(hipMalloc(&h->bcur, (size_t)h->nbk * sizeof(uint32_t)));
-    NIPET_HIP(hipMalloc(&h->gccnt, (size_t)h->ncb * sizeof(uint32_t)));
-    NIPET_HIP(hipMalloc(&h->cstart, (size_t)(h->ncb + 1) * sizeof(uint32_t)));
-    NIPET_HIP(hipMalloc(&h->ccur, (size_t)h->ncb * sizeof(uint32_t)));
-    NIPET_HIP(hipMalloc(&h->fan_part, (size_t)LM_FAN_WG * LM_FAN * sizeof(uint32_t)));
-  }
-  NIPET_HIP(hipMemcpy(h->lut, lut.data(), NSN1 * sizeof(int32_t), hipMemcpyHostToDevice));
-  NIPET_HIP(hipMemcpy(h->rno, c->sn1_rno, NSN1 * sizeof(short2), hipMemcpyHostToDevice));
-  NIPET_HIP(hipMemcpy(h->s2cF, c->s2cF, NSBINANG * sizeof(short2), hipMemcpyHostToDevice));
-  NIPET_HIP(hipMemcpy(h->cdf, cdf, sizeof(cdf), hipMemcpyHostToDevice));
-  int32_t none = -1;
-  NIPET_HIP(hipMemcpy(h->carry, &none, sizeof(int32_t), hipMemcpyHostToDevice));
-  NIPET_HIP(hipMemset(h->bad, 0, sizeof(unsigned int)));
+  LmLayout l{(char *)mem};
+  const int64_t tables = lm_layout(c, h, l);
+  std::vector<char> host(tables, 0);
+  auto put = [&](void *dst, const void *src, size_t n) {
+    std::copy_n((const char *)src, n, host.data() + ((char *)dst - (char *)mem));
+  };
+  const int32_t none = -1;
+  put(h->ssrb_off, soff.data(), (SEG0 + 1) * sizeof(int32_t));
+  put(h->ssrb_list, slist.data(), slist.size() * sizeof(int32_t));
+  put(h->lut, lut.data(), NSN1 * sizeof(int32_t));
+  put(h->rno, c->sn1_rno, NSN1 * sizeof(short2));
+  put(h->s2cF, c->s2cF, NSBINANG * sizeof(short2));
+  put(h->cdf, cdf, sizeof(cdf));
+  put(h->carry, &none, sizeof(none));
   int64_t nf = (int64_t)c->nitag * NBUCKTS;
-  k_fill_u64<<<(int)std::min<int64_t>((nf + 255) / 256, 4096), 256>>>(h->first_nz, ~0ull, nf);
+  k_fill_u64<<<(int)std::min<int64_t>((nf + 255) / 256, 4096), 256, 0, st>>>(h->first_nz, ~0ull,
+                                                                             nf);
   NIPET_HIP(hipGetLastError());
-  NIPET_HIP(hipDeviceSynchronize());
+  // (complete, so that any stream may use the session)
+  NIPET_HIP(hipMemcpyWithStream(mem, host.data(), tables, hipMemcpyHostToDevice, st));
+  NIPET_HIP(hipStreamSynchronize(st));
   return NIPET_OK;
 }
 
@@ -1273,11 +1304,7 @@ __global__ __launch_bounds__(1024) void k_lm_suffix_min(unsigned long long *firs
 
 extern "C" {
 
-int nipet_lm_create(const NipetLmConfig *c, NipetLm **out) {
-  if (!c || !out || !c->sn1_sn11 || !c->sn1_ssrb || !c->sn1_rno || !c->s2cF) {
-    set_error("nipet_lm_create: NULL argument");
-    return NIPET_EINVAL;
-  }
+static int lm_check(const NipetLmConfig *c) {
   if (c->nitag <= 0 || c->tstart < 0 || c->tstop < c->tstart || c->tstop > c->nitag ||
       (c->span != 11 && c->span != 1 && c->span != 0) || c->btp < 0 || c->btp > 2 ||
       c->nrep < 1 || c->nrep > LM_MAXREP || c->rep0 < 0 || c->rep0 > (1 << 30) ||
@@ -1286,9 +1313,41 @@ int nipet_lm_create(const NipetLmConfig *c, NipetLm **out) {
               "nrep=%d)", c->nitag, c->tstart, c->tstop, c->span, c->btp, c->nrep);
     return NIPET_EINVAL;
   }
+  return NIPET_OK;
+}
+
+int64_t nipet_lm_bytes(const NipetLmConfig *c) {
+  if (!c || lm_check(c)) return 0;
+  NipetLm h;
+  LmLayout l{nullptr};
+  lm_layout(c, &h, l);
+  return l.bytes;
+}
+
+int nipet_lm_create_in(const NipetLmConfig *c, void *mem, int64_t bytes, void *stream,
+                       NipetLm **out) {
+  if (!c || !out || !c->sn1_sn11 || !c->sn1_ssrb || !c->sn1_rno || !c->s2cF) {
+    set_error("nipet_lm_create: NULL argument");
+    return NIPET_EINVAL;
+  }
+  int rc = lm_check(c);
+  if (rc) return rc;
+  const int64_t need = nipet_lm_bytes(c);
+  if (mem && (bytes < need || (uintptr_t)mem % 256)) {
+    set_error("nipet_lm_create: memory of %lld bytes, aligned to 256, is needed",
+              (long long)need);
+    return NIPET_EINVAL;
+  }
   NipetLm *h = new NipetLm();
   h->cfg = *c;
-  int rc = lm_build(c, h);
+  if (!mem) {
+    hipError_t e = hipMalloc(&h->own, need);
+    if (e != hipSuccess) {
+      delete h;
+      return hip_fail(e, "nipet_lm_create: hipMalloc");
+    }
+  }
+  rc = lm_build(c, h, mem ? mem : h->own, (hipStream_t)stream);
   if (rc) {
     lm_free(h);
     delete h;
@@ -1296,6 +1355,10 @@ int nipet_lm_create(const NipetLmConfig *c, NipetLm **out) {
   }
   *out = h;
   return NIPET_OK;
+}
+
+int nipet_lm_create(const NipetLmConfig *c, NipetLm **out) {
+  return nipet_lm_create_in(c, nullptr, 0, nullptr, out);
 }
 
 void nipet_lm_destroy(NipetLm *h) {
@@ -1345,8 +1408,48 @@ static int grow(NipetLm *h, int64_t nblk) {
   return NIPET_OK;
 }
 
+// singles list: at most one entry per word; sized generously for the chunk,
+// entries beyond the capacity are reported as an error
+static unsigned int lm_sgl_cap(const NipetLm *h, int64_t n) {
+  const int64_t cap = std::min<int64_t>(std::max<int64_t>(n / 32, 1 << 20), 1 << 28);
+  return std::max((unsigned int)cap, h->sgl_used);  // (never less than for an earlier chunk)
+}
+// one replicate without resampling: sinogram counts privatised in LDS per
+// bucket (staged events need a slot per word of the chunk)
+static bool lm_bin(const NipetLm *h, int64_t n) { return h->gcnt && n <= (int64_t)UINT32_MAX; }
+
+struct LmWork {
+  int32_t *blk_last, *blk_carry;
+  unsigned long long *sgl_idx;
+  int32_t *sgl_word, *sgl_ms;
+  uint32_t *stage, *stage2;
+};
+static int64_t lm_work(const NipetLm *h, int64_t n, void *mem, LmWork &w) {
+  LmLayout l{(char *)mem};
+  const int64_t nblk = (n + LM_BLOCK - 1) / LM_BLOCK, cap = lm_sgl_cap(h, n);
+  w.blk_last = l.take<int32_t>(nblk);
+  w.blk_carry = l.take<int32_t>(nblk);
+  w.sgl_idx = l.take<unsigned long long>(cap);
+  w.sgl_word = l.take<int32_t>(cap);
+  w.sgl_ms = l.take<int32_t>(cap);
+  const int64_t slots = lm_bin(h, n) ? n : 0;
+  w.stage = l.take<uint32_t>(slots);
+  w.stage2 = l.take<uint32_t>(slots);
+  return l.bytes;
+}
+
+int64_t nipet_lm_work_bytes(const NipetLm *h, int64_t n) {
+  LmWork w;
+  return h && n > 0 ? lm_work(h, n, nullptr, w) : 0;
+}
+
 int nipet_lm_chunk(NipetLm *h, const int32_t *words, int64_t n, const NipetLmOut *o,
                    void *stream) {
+  return nipet_lm_chunk_in(h, words, n, o, nullptr, 0, stream);
+}
+
+int nipet_lm_chunk_in(NipetLm *h, const int32_t *words, int64_t n, const NipetLmOut *o,
+                      void *work, int64_t bytes, void *stream) {
   if (!h || !o || (!words && n > 0) || n < 0) {
     set_error("nipet_lm_chunk: bad argument");
     return NIPET_EINVAL;
@@ -1376,17 +1479,24 @@ int nipet_lm_chunk(NipetLm *h, const int32_t *words, int64_t n, const NipetLmOut
     set_error("nipet_lm_chunk: chunk too large");
     return NIPET_EINVAL;
   }
-  // singles list: at most one entry per word; size it generously for the
-  // chunk, entries beyond the capacity are reported as an error
-  unsigned int cap = (unsigned int)std::min<int64_t>(std::max<int64_t>(n / 32, 1 << 20), 1 << 28);
-  // one replicate without resampling: sinogram counts privatised in LDS per
-  // bucket (staged events need a slot per word of the chunk)
-  const bool bin = h->gcnt && n <= (int64_t)UINT32_MAX;
-  int rc = grow(h, nblk);
-  if (rc) return rc;
+  const unsigned int cap = lm_sgl_cap(h, n);
+  const bool bin = lm_bin(h, n);
+  LmWork w = {};
+  int rc = NIPET_OK;
+  if (work) {
+    if (bytes < lm_work(h, n, work, w) || (uintptr_t)work % 256) {
+      set_error("nipet_lm_chunk: work memory of %lld bytes, aligned to 256, is needed",
+                (long long)nipet_lm_work_bytes(h, n));
+      return NIPET_EINVAL;
+    }
+  } else {
+    if ((rc = grow(h, nblk))) return rc;
+    w.blk_last = h->blk_last;
+    w.blk_carry = h->blk_carry;
+  }
   prof_begin(PK_HIST, st);
-  k_lm_tags<<<(unsigned)nblk, LM_THREADS, 0, st>>>(words, n, h->blk_last, h->sgl_count);
-  k_lm_carry<<<1, 1024, 0, st>>>(h->blk_last, h->blk_carry, (int)nblk, h->carry);
+  k_lm_tags<<<(unsigned)nblk, LM_THREADS, 0, st>>>(words, n, w.blk_last, h->sgl_count);
+  k_lm_carry<<<1, 1024, 0, st>>>(w.blk_last, w.blk_carry, (int)nblk, h->carry);
   LmDev p = {};  // singles list and staging slots are set once allocated
   p.words = words;
   p.n = n;
@@ -1406,7 +1516,7 @@ int nipet_lm_chunk(NipetLm *h, const int32_t *words, int64_t n, const NipetLmOut
   p.rno = h->rno;
   p.s2cF = h->s2cF;
   p.cdf = h->cdf;
-  p.blk_carry = h->blk_carry;
+  p.blk_carry = w.blk_carry;
   p.psino = o->psino;
   p.dsino = o->dsino;
   p.ssr = o->ssr;
@@ -1439,16 +1549,22 @@ int nipet_lm_chunk(NipetLm *h, const int32_t *words, int64_t n, const NipetLmOut
     k_lm_bin_scan<<<1, 1024, 0, st>>>(h->gccnt, h->ncb, h->cstart, h->ccur);
   }
   // the tag carry has advanced: a failure from here on ends the session
-  rc = grow_late(h, cap, bin ? n : 0);
-  if (rc) {
-    h->broken = true;
-    return rc;
+  if (!work) {
+    if ((rc = grow_late(h, cap, bin ? n : 0))) {
+      h->broken = true;
+      return rc;
+    }
+    w.sgl_idx = h->sgl_idx;
+    w.sgl_word = h->sgl_word;
+    w.sgl_ms = h->sgl_ms;
+    w.stage = h->stage;
+    w.stage2 = h->stage2;
   }
-  p.sgl_idx = h->sgl_idx;
-  p.sgl_word = h->sgl_word;
-  p.sgl_ms = h->sgl_ms;
-  p.sgl_cap = h->sgl_cap;
-  p.stage = bin ? h->stage : nullptr;
+  p.sgl_idx = w.sgl_idx;
+  p.sgl_word = w.sgl_word;
+  p.sgl_ms = w.sgl_ms;
+  p.sgl_cap = h->sgl_used = cap;
+  p.stage = bin ? w.stage : nullptr;
   p.stage_cap = bin ? n : 0;
   if (c.btp == 1) {
     if (c.nrep == 1)
@@ -1458,8 +1574,8 @@ int nipet_lm_chunk(NipetLm *h, const int32_t *words, int64_t n, const NipetLmOut
   } else if (bin) {
     k_lm_hist<false, false, true><<<(unsigned)nblk, LM_THREADS, 0, st>>>(p);
     k_lm_bin_part<<<(unsigned)((n + LM_TILE - 1) / LM_TILE), LM_THREADS, 0, st>>>(
-        h->stage, h->cstart, h->ncb, h->nbk, h->bcur, h->stage2);
-    k_lm_bin_apply<<<(unsigned)h->nbk, 1024, 0, st>>>(h->stage2, h->bstart, h->nbins, o->psino,
+        w.stage, h->cstart, h->ncb, h->nbk, h->bcur, w.stage2);
+    k_lm_bin_apply<<<(unsigned)h->nbk, 1024, 0, st>>>(w.stage2, h->bstart, h->nbins, o->psino,
                                                        o->dsino);
     if (!merged)
       k_lm_fan<false><<<(unsigned)nwg, LM_THREADS * LM_FAN_SUB, 0, st>>>(p, nblk, h->fan_part, 0,
@@ -1470,10 +1586,10 @@ int nipet_lm_chunk(NipetLm *h, const int32_t *words, int64_t n, const NipetLmOut
   } else {
     k_lm_hist<true, false><<<(unsigned)nblk, LM_THREADS, 0, st>>>(p);
   }
-  k_lm_sgl_first<<<256, 256, 0, st>>>(h->sgl_idx, h->sgl_word, h->sgl_ms, h->sgl_count,
-                                      h->sgl_cap, c.nitag, h->first_nz);
-  k_lm_sgl_apply<<<256, 256, 0, st>>>(h->sgl_idx, h->sgl_word, h->sgl_ms, h->sgl_count,
-                                      h->sgl_cap, c.nitag, h->first_nz, o->bck);
+  k_lm_sgl_first<<<256, 256, 0, st>>>(w.sgl_idx, w.sgl_word, w.sgl_ms, h->sgl_count,
+                                      p.sgl_cap, c.nitag, h->first_nz);
+  k_lm_sgl_apply<<<256, 256, 0, st>>>(w.sgl_idx, w.sgl_word, w.sgl_ms, h->sgl_count,
+                                      p.sgl_cap, c.nitag, h->first_nz, o->bck);
   prof_end(PK_HIST, st);
   NIPET_HIP(hipGetLastError());
   h->base += n;
@@ -1506,7 +1622,7 @@ int nipet_lm_status(NipetLm *h, int64_t *words_done, unsigned int *bad_words,
   NIPET_HIP(hipMemcpy(&cnt, h->sgl_count, sizeof(cnt), hipMemcpyDeviceToHost));
   if (words_done) *words_done = h->base;
   if (bad_words) *bad_words = bad;
-  if (singles_overflow) *singles_overflow = cnt > h->sgl_cap ? cnt - h->sgl_cap : 0;
+  if (singles_overflow) *singles_overflow = cnt > h->sgl_used ? cnt - h->sgl_used : 0;
   return NIPET_OK;
 }
 

@@ -98,7 +98,13 @@ class LmHistogram:
                                  int(self.btp), float(self.btprt), int(seed), self.nrep,
                                  int(rep0), *[k.ctypes.data for k in self._keep])
         h = ct.c_void_p()
-        _lib.check(_lib.lib().nipet_lm_create(ct.byref(cfg), ct.byref(h)), 'nipet_lm_create')
+        # device memory from torch's allocator, which keeps it between sessions
+        self._stream = torch.cuda.current_stream()
+        self._mem = torch.empty(_lib.lib().nipet_lm_bytes(ct.byref(cfg)), dtype=torch.uint8,
+                                device='cuda')
+        _lib.check(_lib.lib().nipet_lm_create_in(
+            ct.byref(cfg), self._mem.data_ptr() or None, self._mem.numel(),
+            self._stream.cuda_stream, ct.byref(h)), 'nipet_lm_create')
         self.handle = h
         z = dict(dtype=torch.int32, device='cuda')
         nb = self.nsinos * 86688
@@ -128,14 +134,24 @@ class LmHistogram:
         if words.dtype != torch.int32 or not words.is_cuda:
             raise TypeError('words must be a CUDA int32 tensor')
         words = words.contiguous()
-        _lib.check(_lib.lib().nipet_lm_chunk(self.handle, words.data_ptr(), words.numel(),
-                                             ct.byref(self._o), _lib.stream_handle()),
-                   'nipet_lm_chunk')
+        n = words.numel()
+        work = torch.empty(_lib.lib().nipet_lm_work_bytes(self.handle, n), dtype=torch.uint8,
+                           device='cuda')
+        _lib.check(_lib.lib().nipet_lm_chunk_in(
+            self.handle, words.data_ptr(), n, ct.byref(self._o), work.data_ptr() or None,
+            work.numel(), self._on_stream()), 'nipet_lm_chunk')
 
     def finish(self):
         """Derive the SSRB prompt sinogram; call after the last chunk."""
         _lib.check(_lib.lib().nipet_lm_finish(self.handle, ct.byref(self._o),
-                                              _lib.stream_handle()), 'nipet_lm_finish')
+                                              self._on_stream()), 'nipet_lm_finish')
+
+    def _on_stream(self):
+        """Handle of the current stream, which the session's memory outlives."""
+        st = _torch().cuda.current_stream()
+        if st != self._stream:
+            self._mem.record_stream(st)
+        return st.cuda_stream
 
     def status(self):
         n, bad, ovf = ct.c_int64(), ct.c_uint(), ct.c_uint()
