@@ -258,25 +258,30 @@ struct LmHead {
   unsigned long long z = 0;
 };
 
+// (replicate r of nr: the centre-of-mass sums are those of r = 0)
 __device__ inline void lm_head_flush(LmHead &h, int itag0, uint32_t *hcp, uint32_t *hcd,
                                      unsigned long long *mzr, unsigned long long *mzm,
-                                     const LmDev &p) {
+                                     const LmDev &p, int nr = 1, int r = 0) {
   if (h.p | h.d) {
     const int it = itag0 + h.k;
     if (h.k >= 0 && h.k < LM_HW) {
       if (h.p) {
-        atomicAdd(&hcp[h.k], h.p);
-        atomicAdd(&mzr[h.k], h.z);
-        atomicAdd(&mzm[h.k], (unsigned long long)h.p);
+        atomicAdd(&hcp[h.k * nr + r], h.p);
+        if (r == 0) {
+          atomicAdd(&mzr[h.k], h.z);
+          atomicAdd(&mzm[h.k], (unsigned long long)h.p);
+        }
       }
-      if (h.d) atomicAdd(&hcd[h.k], h.d);
+      if (h.d) atomicAdd(&hcd[h.k * nr + r], h.d);
     } else {
       if (h.p) {
-        atomicAdd(p.phc + it, h.p);
-        atomicAdd(p.zR + it, h.z);
-        atomicAdd(p.zM + it, (unsigned long long)h.p);
+        atomicAdd(p.phc + (int64_t)it * nr + r, h.p);
+        if (r == 0) {
+          atomicAdd(p.zR + it, h.z);
+          atomicAdd(p.zM + it, (unsigned long long)h.p);
+        }
       }
-      if (h.d) atomicAdd(p.dhc + it, h.d);
+      if (h.d) atomicAdd(p.dhc + (int64_t)it * nr + r, h.d);
     }
   }
   h.p = h.d = 0;
@@ -287,9 +292,9 @@ __device__ inline void lm_head_flush(LmHead &h, int itag0, uint32_t *hcp, uint32
 __device__ inline void lm_head_add(LmHead &h, uint32_t hp, uint32_t hz, uint32_t hd, int k,
                                    int itag0, uint32_t *hcp, uint32_t *hcd,
                                    unsigned long long *mzr, unsigned long long *mzm,
-                                   const LmDev &p) {
+                                   const LmDev &p, int nr = 1, int r = 0) {
   if (k != h.k) {
-    lm_head_flush(h, itag0, hcp, hcd, mzr, mzm, p);
+    lm_head_flush(h, itag0, hcp, hcd, mzr, mzm, p, nr, r);
     h.k = k;
   }
   h.p += hp;
@@ -298,7 +303,13 @@ __device__ inline void lm_head_add(LmHead &h, uint32_t hp, uint32_t hz, uint32_t
 }
 
 // REP = false: one event per lane (nrep == 1).
-// REP = true: the wave walks its events one by one, lane r = replicate r.
+// REP = true: nr replicates share a group of lanes (the next power of two), lane
+// r of it = replicate r, and the wave's groups walk its words a quad each: one
+// generator call serves the quad's four words, and 64 / 16 quads at a time for 16
+// replicates. Each lane decodes its own word once, into LDS, from where the
+// groups read it. Bound by the generator's 32-bit products and the random
+// 64-byte atomics: one event at a time on nr of 64 lanes took 9.8 ms for 60 M
+// words and 16 replicates, now 4.2 (the generator about 1 ms of it).
 // NP: non-parametric bootstrap (btp = 1): the block's event words are
 // compacted in word order into LDS (the resampling patch) and every counted
 // event is replaced by a draw from them.
@@ -321,6 +332,9 @@ __global__ __launch_bounds__(LM_THREADS) void k_lm_hist(LmDev p) {
   __shared__ int32_t wave_last[LM_WAVES];
   __shared__ uint32_t crank[BIN ? LM_MAXCB : 1], cbase[BIN ? LM_MAXCB : 1];
   __shared__ uint32_t stg[BIN ? LM_BLOCK : 1];  // the block's staged events, by coarse bucket
+  // REP: the decoded words of each wave (bin or -1, second | prompt << 30, and
+  // the two fields of k_lm_hist's other outputs)
+  __shared__ int4 dec[REP && !NP ? LM_THREADS : 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nr = REP ? p.nrep : 1;
   for (int i = tid; i < NSN1; i += LM_THREADS) lut[i] = p.lut[i];
@@ -377,10 +391,11 @@ __global__ __launch_bounds__(LM_THREADS) void k_lm_hist(LmDev p) {
   }
 
   const unsigned long long le = (lane == 63) ? ~0ull : ((2ull << lane) - 1);
-  // REP: the last generator call of the wave (its word quad, the 4 draws)
-  uint64_t bq = ~0ull;
-  uint32_t bc[4] = {0u, 0u, 0u, 0u};
-  LmHead hs;  // one replicate: this lane's head-curve sums
+  // REP: lane groups of 2^gsh lanes, this lane's replicate and group
+  int gsh = 0;
+  while (REP && (1 << gsh) < nr) gsh++;
+  const int rep = lane & ((1 << gsh) - 1), grp = lane >> gsh;
+  LmHead hs;  // this lane's head-curve sums (one replicate)
   // BIN: each word's staged value and coarse bucket (16 bits each, two per
   // register; 0xffff: not counted), kept until the block's runs are laid out
   uint32_t bpay[BIN ? LM_PER_LANE : 1], bcb[BIN ? LM_PER_LANE / 2 : 1];
@@ -525,10 +540,7 @@ __global__ __launch_bounds__(LM_THREADS) void k_lm_hist(LmDev p) {
         }
       }
     } else {
-      // Each lane decodes its own word once (VALU); the loop over the wave's
-      // events then broadcasts the decoded fields with readlane, so the
-      // scalar unit only walks the event mask.
-      int32_t e_addr = 0, e_x1 = 0, e_x2 = -1;
+      int4 e = make_int4(-1, 0, 0, -1);
       if (ev) {
         const int32_t v = word & 0x3fffffff;
         const int si = v / NSBINANG, aw = v - si * NSBINANG;
@@ -536,68 +548,66 @@ __global__ __launch_bounds__(LM_THREADS) void k_lm_hist(LmDev p) {
         const int32_t lu = lut[si];
         const int s11 = lu >> 16, sr = lu & 0xffff;
         // bin address (< 4084 * 86688 < 2^31)
-        e_addr = p.span == 11 ? s11 * NSBINANG + aw : (p.span == 1 ? v : sr * NSBINANG + aw);
+        e.x = p.span == 11 ? s11 * NSBINANG + aw : (p.span == 1 ? v : sr * NSBINANG + aw);
+        e.y = itag | (word & (1 << 30));
         if ((word >> 30) & 1) {
           // prompt: SSRB plane (centre of mass), projection-view offset with
           // bit 30 set for the second view (a = 126), -1 for none
-          e_x1 = sr;
+          e.z = sr;
           if ((a == 0 || a == 126) && itag < MXNITAG)
-            e_x2 = ((itag >> VTIME) * SEG0 * NSBINS + sr * NSBINS + w) | ((a == 126) << 30);
+            e.w = ((itag >> VTIME) * SEG0 * NSBINS + sr * NSBINS + w) | ((a == 126) << 30);
         } else {
           // delayed: the two fan-sum entries
           const short2 rr = p.rno[si], cr = p.s2cF[a + NSANGLES * w];
-          e_x1 = NCRS * rr.x + cr.x;
-          e_x2 = NCRS * rr.y + cr.y;
+          e.z = NCRS * rr.x + cr.x;
+          e.w = NCRS * rr.y + cr.y;
         }
       }
-      unsigned long long evm = __ballot(ev);
-      while (evm) {
-        const int l = __ffsll((long long)evm) - 1;
-        evm &= evm - 1;
-        const int32_t wv = __builtin_amdgcn_readlane(word, l);
-        const int it = __builtin_amdgcn_readlane(itag, l);
-        const int32_t addr = __builtin_amdgcn_readlane(e_addr, l);
-        const int32_t x1 = __builtin_amdgcn_readlane(e_x1, l);
-        const int32_t x2 = __builtin_amdgcn_readlane(e_x2, l);
-        const uint64_t g = (uint64_t)(p.base + w0 + j * 64 + l);
-        uint32_t N = lane < nr ? 1u : 0u;
-        if (p.btp == 2) {
-          if ((g >> 2) != bq) {  // wave-uniform: one generator call per quad of words
-            bq = g >> 2;
-            boot_quad(bc, g, (uint32_t)(p.rep0 + lane), p.k0, p.k1);
-          }
-          const uint32_t n0 = poisson_n(boot_pick(bc, g), c8, cdf);
-          N = lane < nr ? n0 : 0u;
+      if (!__ballot(ev)) continue;
+      dec[wave * 64 + lane] = e;
+      __builtin_amdgcn_wave_barrier();
+      // quads of the session's words: the first and the last may be partial
+      const uint64_t g0 = (uint64_t)(p.base + w0 + j * 64);
+      const int lead = (int)(g0 & 3), nq = (64 + lead + 3) >> 2;
+      for (int q0 = 0; q0 < nq; q0 += 64 >> gsh) {
+        const int q = q0 + grp, l0 = 4 * q - lead;
+        int4 d[4];
+        bool any = false;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          const int l = l0 + t;
+          d[t] = dec[wave * 64 + min(max(l, 0), 63)];
+          if (l < 0 || l > 63 || rep >= nr) d[t].x = -1;
+          any |= d[t].x >= 0;
         }
-        const bool ok = N > 0 && N < 32;
-        const int k = it - itag0;
-        const bool inwin = k >= 0 && k < LM_HW;
-        const bool prompt = (wv >> 30) & 1;
-        if (ok) {
-          atomicAdd((prompt ? p.psino : p.dsino) + (int64_t)addr * nr + lane, N);
-          uint32_t *hl = prompt ? hcp : hcd;
-          uint32_t *hg = prompt ? p.phc : p.dhc;
-          if (inwin) atomicAdd(&hl[k * nr + lane], N); else atomicAdd(hg + (int64_t)it * nr + lane, N);
-        }
-        if (lane == 0 && ok) {
-          if (prompt) {
-            if (inwin) {
-              atomicAdd(&mzr[k], (unsigned long long)x1);
-              atomicAdd(&mzm[k], (unsigned long long)N);
+        if (!__ballot(any)) continue;
+        uint32_t bc[4];
+        if (p.btp == 2)  // wave-uniform
+          boot_quad(bc, g0 - lead + 4 * (uint64_t)q, (uint32_t)(p.rep0 + rep), p.k0, p.k1);
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          const uint32_t N = p.btp == 2 ? poisson_n(bc[t], c8, cdf) : 1u;
+          if (d[t].x < 0 || N == 0 || N >= 32) continue;
+          const bool prompt = (d[t].y >> 30) & 1;
+          const int it = d[t].y & 0x3fffffff;
+          atomicAdd((prompt ? p.psino : p.dsino) + (int64_t)d[t].x * nr + rep, N);
+          lm_head_add(hs, prompt ? N : 0u, (uint32_t)d[t].z, prompt ? 0u : N, it - itag0, itag0,
+                      hcp, hcd, mzr, mzm, p, nr, rep);
+          if (rep == 0) {
+            if (prompt) {
+              if (d[t].w >= 0)
+                atomicAdd(p.pvs + (d[t].w & 0x3fffffff), N << (8 * ((d[t].w >> 30) & 1)));
             } else {
-              atomicAdd(p.zR + it, (unsigned long long)x1);
-              atomicAdd(p.zM + it, (unsigned long long)N);
+              atomicAdd(p.fan + d[t].z, N);
+              atomicAdd(p.fan + d[t].w, N);
             }
-            if (x2 >= 0) atomicAdd(p.pvs + (x2 & 0x3fffffff), N << (8 * ((x2 >> 30) & 1)));
-          } else {
-            atomicAdd(p.fan + x1, N);
-            atomicAdd(p.fan + x2, N);
           }
         }
       }
+      __builtin_amdgcn_wave_barrier();
     }
   }
-  if (!REP) lm_head_flush(hs, itag0, hcp, hcd, mzr, mzm, p);
+  if (!REP || !NP) lm_head_flush(hs, itag0, hcp, hcd, mzr, mzm, p, nr, REP ? rep : 0);
   if constexpr (BIN) {
     // one run of slots per coarse bucket: crank becomes the run's first slot
     // in stg (exclusive scan by wave 0), cbase the run's global slot minus
