@@ -719,6 +719,26 @@ __global__ void k_lm_ssrb(const uint32_t *psino, int nrep, const int32_t *s_off,
   }
 }
 
+// k_lm_ssrb of one replicate, four bins a thread (16-byte reads, four planes'
+// rows in flight): one bin a thread took 152 us for span 11 (290 MB), now
+// 77.
+__global__ void k_lm_ssrb4(const uint4 *__restrict__ psino, const int32_t *__restrict__ s_off,
+                           const int32_t *__restrict__ s_list, uint4 *__restrict__ ssr) {
+  const int pl = blockIdx.y, i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= NSBINANG / 4) return;
+  uint4 acc = make_uint4(0, 0, 0, 0);
+  const int k1 = s_off[pl + 1];
+#pragma unroll 4
+  for (int k = s_off[pl]; k < k1; k++) {
+    const uint4 v = psino[(int64_t)s_list[k] * (NSBINANG / 4) + i];
+    acc.x += v.x;
+    acc.y += v.y;
+    acc.z += v.z;
+    acc.w += v.w;
+  }
+  ssr[(int64_t)pl * (NSBINANG / 4) + i] = acc;
+}
+
 // Delayed fan-sums of one-replicate sessions (the sessions whose sinogram
 // counts are LDS-privatised). In the event kernel each delayed event's two
 // crystal ends were global atomics into the 64 x 504 fan-sums (about 2 ms of
@@ -822,12 +842,16 @@ __global__ __launch_bounds__(LM_THREADS * LM_FAN_SUB) void k_lm_fan(LmDev p, int
   }
 }
 
+// (LM_FAN_SPLIT blocks share a place's copies: one alone reads 256 in series:
+// 98 us, now 13)
+constexpr int LM_FAN_SPLIT = 16;
 __global__ void k_lm_fan_sum(const uint32_t *__restrict__ part, int nwg, uint32_t *fan) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= LM_FAN) return;
-  uint32_t acc = 0;
-  for (int b = 0; b < nwg; b++) acc += part[(int64_t)b * LM_FAN + i];
-  fan[i] += acc;
+  uint32_t s = 0;
+#pragma unroll 8
+  for (int k = blockIdx.y; k < nwg; k += LM_FAN_SPLIT) s += part[(size_t)k * LM_FAN + i];
+  if (s) atomicAdd(fan + i, s);
 }
 
 __global__ void k_fill_u64(unsigned long long *p, unsigned long long v, int64_t n) {
@@ -1035,15 +1059,13 @@ __global__ __launch_bounds__(LM_THREADS) void k_lm_bin_part(const uint32_t *__re
 __global__ __launch_bounds__(1024) void k_lm_bin_apply(const uint32_t *__restrict__ stage,
                                                        const uint32_t *__restrict__ bstart,
                                                        int64_t nbins, uint32_t *psino,
-                                                       uint32_t *dsino) {
-  __shared__ uint32_t pc[LM_BBINS], dc[LM_BBINS];
+                                                       uint32_t *dsino, int vec) {
+  __shared__ __align__(16) uint32_t pc[LM_BBINS], dc[LM_BBINS];
   const int tid = threadIdx.x;
   const uint32_t s0 = bstart[blockIdx.x], s1 = bstart[blockIdx.x + 1];
   if (s0 == s1) return;  // block-uniform, before any barrier
-  for (int i = tid; i < LM_BBINS; i += 1024) {
-    pc[i] = 0;
-    dc[i] = 0;
-  }
+  for (int i = tid; i < LM_BBINS / 4; i += 1024)
+    ((uint4 *)pc)[i] = ((uint4 *)dc)[i] = make_uint4(0, 0, 0, 0);
   __syncthreads();
   // eight loads in flight per thread before their counts
   constexpr int PER = 8;
@@ -1063,6 +1085,30 @@ __global__ __launch_bounds__(1024) void k_lm_bin_apply(const uint32_t *__restric
   __syncthreads();
   const int64_t base = (int64_t)blockIdx.x << LM_BSHIFT;
   const int lim = (int)(nbins - base < LM_BBINS ? nbins - base : LM_BBINS);
+  // 16-byte groups (bins come in fours), all of a thread's reads before its adds:
+  // one workgroup's LDS fills a CU, and 32 read-adds in series took 360 us of a
+  // 10 s frame's kernels (10 M words), now 140
+  if (vec) {
+    constexpr int G = LM_BBINS / 4096;
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+      const uint4 *c = (const uint4 *)(a ? dc : pc);
+      uint4 *o = (uint4 *)((a ? dsino : psino) + base);
+      uint4 n[G], v[G];
+#pragma unroll
+      for (int k = 0; k < G; k++) {
+        const int i = tid + k * 1024;
+        n[k] = 4 * i < lim ? c[i] : make_uint4(0, 0, 0, 0);
+        if (n[k].x | n[k].y | n[k].z | n[k].w) v[k] = o[i];
+      }
+#pragma unroll
+      for (int k = 0; k < G; k++)
+        if (n[k].x | n[k].y | n[k].z | n[k].w)
+          o[tid + k * 1024] = make_uint4(v[k].x + n[k].x, v[k].y + n[k].y, v[k].z + n[k].z,
+                                         v[k].w + n[k].w);
+    }
+    return;
+  }
   for (int i = tid; i < lim; i += 1024) {
     if (pc[i]) psino[base + i] += pc[i];
     if (dc[i]) dsino[base + i] += dc[i];
@@ -1585,12 +1631,13 @@ int nipet_lm_chunk_in(NipetLm *h, const int32_t *words, int64_t n, const NipetLm
     k_lm_hist<false, false, true><<<(unsigned)nblk, LM_THREADS, 0, st>>>(p);
     k_lm_bin_part<<<(unsigned)((n + LM_TILE - 1) / LM_TILE), LM_THREADS, 0, st>>>(
         w.stage, h->cstart, h->ncb, h->nbk, h->bcur, w.stage2);
+    const int vec = ((uintptr_t)o->psino | (uintptr_t)o->dsino) % 16 == 0 && h->nbins % 4 == 0;
     k_lm_bin_apply<<<(unsigned)h->nbk, 1024, 0, st>>>(w.stage2, h->bstart, h->nbins, o->psino,
-                                                       o->dsino);
+                                                       o->dsino, vec);
     if (!merged)
       k_lm_fan<false><<<(unsigned)nwg, LM_THREADS * LM_FAN_SUB, 0, st>>>(p, nblk, h->fan_part, 0,
                                                                          nullptr, nullptr);
-    k_lm_fan_sum<<<(LM_FAN + 255) / 256, 256, 0, st>>>(h->fan_part, nwg, o->fan);
+    k_lm_fan_sum<<<dim3((LM_FAN + 255) / 256, LM_FAN_SPLIT), 256, 0, st>>>(h->fan_part, nwg, o->fan);
   } else if (c.nrep == 1) {
     k_lm_hist<false, false><<<(unsigned)nblk, LM_THREADS, 0, st>>>(p);
   } else {
@@ -1615,8 +1662,12 @@ int nipet_lm_finish(NipetLm *h, const NipetLmOut *o, void *stream) {
     set_error("nipet_lm_finish: a chunk of this session failed part-way");
     return NIPET_EINVAL;
   }
-  k_lm_ssrb<<<4096, 256, 0, (hipStream_t)stream>>>(o->psino, h->cfg.nrep, h->ssrb_off,
-                                                     h->ssrb_list, o->ssr);
+  if (h->cfg.nrep == 1 && ((uintptr_t)o->psino | (uintptr_t)o->ssr) % 16 == 0)
+    k_lm_ssrb4<<<dim3((NSBINANG / 4 + 255) / 256, SEG0), 256, 0, (hipStream_t)stream>>>(
+        (const uint4 *)o->psino, h->ssrb_off, h->ssrb_list, (uint4 *)o->ssr);
+  else
+    k_lm_ssrb<<<4096, 256, 0, (hipStream_t)stream>>>(o->psino, h->cfg.nrep, h->ssrb_off,
+                                                       h->ssrb_list, o->ssr);
   NIPET_HIP(hipGetLastError());
   return NIPET_OK;
 }

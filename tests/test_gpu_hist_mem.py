@@ -55,3 +55,26 @@ def test_callers_memory_equals_own(params, words, span, btp, nrep):
     size = L.nipet_lm_bytes(ct.byref(cfg))
     assert L.nipet_lm_create_in(ct.byref(cfg), mem.data_ptr(), size - 1, _lib.stream_handle(),
                                 ct.byref(own)) != 0
+
+
+@pytest.mark.parametrize('span', [11, 0])
+def test_outputs_at_odd_addresses(params, words, span):
+    """Outputs that are not aligned to 16 bytes, in two chunks: the same counts."""
+    import torch
+
+    from nipet_amd.lm.mmrhist import LmHistogram, tag_range
+    tf, tl = tag_range(words)
+    outs = []
+    for shift in (0, 1):
+        h = LmHistogram(params, tf, (tl - tf + 999) // 1000, span=span)
+        for k in ('psino', 'dsino', 'ssr'):
+            t = h.out[k]
+            h.out[k] = torch.zeros(t.numel() + shift, dtype=t.dtype,
+                                   device='cuda')[shift:].view(t.shape)
+            setattr(h._o, k, h.out[k].data_ptr())
+        h.add(words[:5 * 8192])
+        h.add(words[5 * 8192:])
+        h.finish()
+        outs.append(h.out)
+    for k in outs[0]:
+        assert torch.equal(outs[0][k], outs[1][k]), k
