@@ -230,7 +230,7 @@ int nipet_norm_sino(NipetNorm *h, const NipetNormComp *c, const int32_t *buckets
   k_nrm_eff<<<(NRM_NRNG * NRM_NCRS + 255) / 256, 256, 0, st>>>(h->d);
   k_nrm_axial<<<(NRM_NSN1 + 255) / 256, 256, 0, st>>>(h->d);
   k_nrm_tx<<<(h->d.naw + 255) / 256, 256, 0, st>>>(h->d);
-  k_pair_sino<<<pair_blocks(h->d.naw), PAIR_THREADS, 0, st>>>(out, h->ps);
+  launch_pair_sino(out, h->ps, st);
   NIPET_HIP(hipGetLastError());
   return NIPET_OK;
 }

@@ -42,13 +42,15 @@ __global__ void k_rnd_fsum(float *f, const uint32_t *fan, const int16_t *crsri) 
 }
 
 // INIT: so = sqrt(f / F 1) (F 1 = run length x ring-band length);
-// else: so = si / 2 + (F si > 0 ? f / F si : 0) / 2. Block = crystal c, 256
-// threads = 4 partial sums x 64 rings.
+// else: so = si / 2 + (F si > 0 ? f / F si : 0) / 2. Block = crystal c, RND_G
+// partial sums x 64 rings. Bound by the latency of its 320 reads a ring, RND_U
+// in flight: four partial sums, one read at a time, took 15 us, now 6.8.
+constexpr int RND_G = 16, RND_U = 10;
 template <bool INIT>
-__global__ __launch_bounds__(256) void k_rnd_step(float *__restrict__ so,
+__global__ __launch_bounds__(64 * RND_G) void k_rnd_step(float *__restrict__ so,
                                                   const float *__restrict__ si,
                                                   const float *__restrict__ f, RndDev d) {
-  __shared__ float part[4][RND_NR];
+  __shared__ float part[RND_G][RND_NR];
   __shared__ float u[RND_NR];
   const int c = blockIdx.x, g = threadIdx.x >> 6, r = threadIdx.x & 63;
   const short2 run = d.run[c];
@@ -60,18 +62,39 @@ __global__ __launch_bounds__(256) void k_rnd_step(float *__restrict__ so,
     return;
   }
   float acc = 0.f;
-  for (int k = g; k < run.y; k += 4) {
-    int q = run.x + k;
-    if (q >= RND_NC) q -= RND_NC;
-    acc += si[q * RND_NR + r];
+  for (int k0 = g; k0 < run.y; k0 += RND_G * RND_U) {
+    float v[RND_U];
+#pragma unroll
+    for (int u = 0; u < RND_U; u++) {
+      const int k = k0 + u * RND_G;
+      int q = run.x + min(k, run.y - 1);
+      if (q >= RND_NC) q -= RND_NC;
+      v[u] = si[q * RND_NR + r];
+    }
+#pragma unroll
+    for (int u = 0; u < RND_U; u++) acc += k0 + u * RND_G < run.y ? v[u] : 0.f;
   }
   part[g][r] = acc;
   __syncthreads();
-  if (g == 0) u[r] = (part[0][r] + part[1][r]) + (part[2][r] + part[3][r]);
+  if (g == 0) {
+    float t = 0.f;
+#pragma unroll
+    for (int k = 0; k < RND_G; k += 4)
+      t += (part[k][r] + part[k + 1][r]) + (part[k + 2][r] + part[k + 3][r]);
+    u[r] = t;
+  }
   __syncthreads();
   if (g == 0) {
     float fs = 0.f;
-    for (int q = lo; q <= hi; q++) fs += u[q];
+    int q = lo;
+    for (; q + 15 <= hi; q += 16) {  // reads in flight, sums in order
+      float v[16];
+#pragma unroll
+      for (int k = 0; k < 16; k++) v[k] = u[q + k];
+#pragma unroll
+      for (int k = 0; k < 16; k++) fs += v[k];
+    }
+    for (; q <= hi; q++) fs += u[q];
     const float qv = fs > 0.f ? f[i] / fs : 0.f;
     so[i] = 0.5f * si[i] + 0.5f * qv;
   }
@@ -213,14 +236,14 @@ int nipet_rnd_estimate(NipetRnd *h, const uint32_t *fansums, int niter, float *r
   }
   hipStream_t st = (hipStream_t)stream;
   k_rnd_fsum<<<(RND_NR * RND_NCRS + 255) / 256, 256, 0, st>>>(h->f, fansums, h->d.crsri);
-  k_rnd_step<true><<<RND_NC, 256, 0, st>>>(h->s[0], h->s[1], h->f, h->d);
+  k_rnd_step<true><<<RND_NC, 64, 0, st>>>(h->s[0], h->s[1], h->f, h->d);
   int cur = 0;
   for (int k = 0; k < niter; k++, cur ^= 1)
-    k_rnd_step<false><<<RND_NC, 256, 0, st>>>(h->s[cur ^ 1], h->s[cur], h->f, h->d);
+    k_rnd_step<false><<<RND_NC, 64 * RND_G, 0, st>>>(h->s[cur ^ 1], h->s[cur], h->f, h->d);
   if (rsino) {
     PairSino p = h->ps;
     p.tab = h->s[cur];
-    k_pair_sino<<<pair_blocks(p.naw), PAIR_THREADS, 0, st>>>(rsino, p);
+    launch_pair_sino(rsino, p, st);
   }
   if (cmap)
     k_rnd_cmap<<<(RND_NCRS * RND_NR + 255) / 256, 256, 0, st>>>(cmap, h->s[cur], h->d.crsri);
