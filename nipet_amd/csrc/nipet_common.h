@@ -14,7 +14,7 @@ constexpr int NZ = 127;   // device image z (w), fastest
 // segments of one transaxial ray: one per voxel column it crosses, at most
 // one more than the grid lines it crosses (checked when the geometry is built)
 constexpr int MAX_SEG = NX + NY + 1;
-constexpr int SEG_PAD = 64;  // records behind the last list (whole chunks are read)
+constexpr int SEG_PAD = 128;  // records behind the last list (whole chunks are read)
 constexpr int64_t NVOX = (int64_t)NX * NY * NZ;
 constexpr int MAXNSN = 4096;  // largest sinogram count handled (span-1: 4084)
 constexpr int LI_MAX = 2112;  // largest Michelogram (ring pair) count
@@ -65,8 +65,9 @@ struct Geom {
   float *lmax = nullptr;     // [naw] longest segment of the ray
   // z crossings of a ray [naw][ev_off(dmax + 1)]: entry ev_off(d) + w is where
   // the LORs of ring difference d pass from plane offset w to w + 1, at t =
-  // (w + 1/2) atn / (2 d): (segment << 10 | ev_phi(w), distance into the
-  // segment), segment 2^22 - 1 past the end of the list
+  // (w + 1/2) atn / (2 d): how far into its segment, as a fraction in float64,
+  // with its low 20 bits (2^-32 of it) replaced by segment << 10 | ev_phi(w);
+  // segment 1023 past the end of the list
   uint2 *ev = nullptr;
   float2 *li_z = nullptr;    // [nli] (zeta_a at t=0, zeta_b - zeta_a) in z-voxel units
   short2 *li_sn = nullptr;   // [nli] output sinogram of LOR a and of its mirror b
@@ -127,6 +128,8 @@ __device__ inline uint2 bp_event(int d, int w, double beta, bool last) {
 // Position of plane w in the forward projector's LDS rows (64 even planes, then
 // 64 odd ones, of 8 bytes), in bytes.
 __host__ __device__ constexpr int ev_phi(int w) { return ((w & 1) << 9) + ((w >> 1) << 3); }
+constexpr uint32_t EV_PLACE = 0xfffffu;  // the place in an entry of Geom::ev
+static_assert(MAX_SEG < 1023, "segments in 10 bits");
 // Crossings of ring difference d in Geom::ev: 2 d, and eight that lie past any
 // segment (eight are read at a time).
 __host__ __device__ constexpr int ev_off(int d) { return (d - 1) * (d + 8); }

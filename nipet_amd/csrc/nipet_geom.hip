@@ -258,12 +258,15 @@ __global__ __launch_bounds__(256) void k_events(const int32_t *__restrict__ off,
       const int m = (lo + hi) >> 1;
       if (s[m] <= t) lo = m; else hi = m;
     }
-    uint2 e = make_uint2(~0u, 0u);
-    if (n > 0) {
-      const float len = seg[beg + lo].len;
-      if (w < 2 * d && (lo < n - 1 || t < s[lo] + (double)len))
-        e.x = ((unsigned)lo << 10) | (unsigned)ev_phi(w);
-      e.y = __float_as_uint(fminf(fmaxf((float)(t - s[lo]), 0.f), len));
+    uint2 e = make_uint2(EV_PLACE, 0u);
+    if (n > 0 && w < 2 * d) {
+      const double len = seg[beg + lo].len;
+      if (lo < n - 1 || t < s[lo] + len) {
+        const double f = len > 0.0 ? fmin(fmax((t - s[lo]) / len, 0.0), 1.0) : 0.0;
+        const unsigned long long b = (unsigned long long)__double_as_longlong(f);
+        e = make_uint2(((unsigned)b & ~EV_PLACE) | (unsigned)lo << 10 | (unsigned)ev_phi(w),
+                       (unsigned)(b >> 32));
+      }
     }
     ev[(size_t)aw * ne + i] = e;
   }

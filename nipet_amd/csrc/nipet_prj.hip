@@ -138,41 +138,52 @@ __device__ inline double rdlane(double v, int l) {
 //   C_{2 d - w_end + 2 r0}(t_end) - sum_w [C_p - C_{p + 1}](t_w), p = 2 d - w - 1 + 2 r0.
 // The work is therefore one LDS read per z crossing (about 1.8 d per LOR, 37
 // on average), not one per voxel segment (272 on average): a subset of 4,894
-// bins takes 0.56 ms against 0.95 by segments, all 68,516 bins 7.4 against
-// 12.6; two images 0.49 ms each against 0.71 in fours. VALU issue is at 0.67
-// of its limit, LDS at 0.45, and about half of both goes to staging.
-//  - Chunks of FZ_CH segments: E[j][p] = (C_p - C_{p + 1}) at the start of
-//    segment j as a float64 prefix sum over the whole ray and D[j][p] =
-//    I_p - I_{p + 1} of the segment's voxel column as float32; a crossing at
-//    distance a into segment j adds E[j][p] + a D[j][p]. The sums telescope
-//    over planes the LOR never enters, so they are kept in float64, which
-//    costs no more instructions than float32 on this chip (full-rate FP64);
-//    a LOR that misses the object is left with rounding of 1e-16 of the
-//    bin's largest line integral and is set to 0 (FZ_SNAP).
+// bins takes 0.50 ms against 0.95 by segments, all 68,516 bins 6.7 against
+// 12.6. VALU, scalar unit and LDS are each at 0.6 of their limits: what is left
+// is waves waiting for their turn at all three.
+//  - Rows E[j][p] = (C_p - C_{p + 1}) at the start of segment j, a float64
+//    prefix sum along the ray, in a ring of FZ_RING rows; a crossing at the
+//    fraction f of segment j adds E[j][p] + f (E[j + 1][p] - E[j][p]): one
+//    16-byte LDS read. The sums telescope over planes the LOR never enters, so
+//    they are kept in float64, which costs no more instructions than float32 on
+//    this chip (full-rate FP64); a LOR that misses the object is left with
+//    rounding of 1e-16 of the bin's largest line integral and is set to 0
+//    (FZ_SNAP).
+//  - Two waves stage the rows of a chunk of FZ_CH segments while the others
+//    cross the chunk before: one barrier a chunk, and no wave does both. The
+//    staging waves wait for memory, so a whole chunk of columns is on its way
+//    (one register a row: lane = plane, the next plane from the next lane).
+//    All waves staging, then all crossing, with the chunk's totals exchanged:
+//    0.56 ms; two planes a lane and half a chunk on its way: 0.55.
 //  - Lanes: half a wave is 32 LORs (r0 = lane, lane + 32), the other half
 //    their mirrors; the crossing is wave-uniform. Rows hold the even planes
 //    and then the odd ones, so the 32 lanes of a half read consecutive
 //    words: no bank conflicts at any d.
-//  - Waves: wave v owns the ring differences 63 - v, 32 + v, 31 - v and v:
-//    the same number of crossings for every v (but for those above dmax).
-//    From d = 32 on only rings r0 < 32 start a LOR. Where a crossing lies
-//    (segment, distance) is geometry: the table Geom::ev, read through the
-//    scalar cache two crossings ahead (the vector unit is the busiest one).
+//  - The crossing waves take the ring differences from the largest down in
+//    turns, so that each has about the same number of crossings. From d = 32 on
+//    only rings r0 < 32 start a LOR. Where a crossing lies (segment, fraction)
+//    is geometry: the table Geom::ev, read through the scalar cache (the vector
+//    unit has enough to do).
 //  - Non-finite voxels: a prefix sum would carry them into LORs that do not
 //    touch them. A bin whose totals are not finite is walked segment by
 //    segment instead.
 // Span-1 -> span-N: each output bin sums its LORs in a fixed order from LDS
 // (no atomics, bit-reproducible).
 constexpr int FZ_THREADS = 1024;
-constexpr int FZ_NG = FZ_THREADS / 128;    // groups of 128 threads (2 waves: even / odd planes)
-constexpr int FZ_RPG = 4;                  // rows staged per group
-constexpr int FZ_CH = FZ_NG * FZ_RPG;      // segments per chunk
-constexpr int FZ_NS = 4;                   // ring differences per wave (16 waves x 4 = 64)
-constexpr int FZ_NE = FZ_CH * 128 + 64;    // lanes past ring 63 read behind the last row
+constexpr int FZ_SW = 2;                   // staging waves (planes 0 .. 62, 63 .. 126)
+constexpr int FZ_CW = FZ_THREADS / 64 - FZ_SW;  // crossing waves
+constexpr int FZ_CH = 30;                  // segments per chunk
+constexpr int FZ_PF = FZ_CH;               // columns read ahead by a staging wave
+constexpr int FZ_NS = 6;                   // ring differences per crossing wave
+constexpr int FZ_RING = 64;                // rows in LDS, by segment modulo FZ_RING
+// the ring, its first row again (the row behind the last), and what lanes past
+// ring 63 read (the last of it: where a lane without a plane writes)
+constexpr int FZ_NE = (FZ_RING + 1) * 128 + 64;
 constexpr double FZ_SNAP = 0x1p-44;
-static_assert(FZ_CH <= SEG_PAD, "whole chunks of records are read");
+static_assert(2 * FZ_CH + 1 <= FZ_RING, "a chunk is staged while the one before is read");
+static_assert(3 * FZ_CH <= SEG_PAD, "records behind the list are read");
 static_assert(FZ_NE * sizeof(double) >= (2 * LI_MAX + 1) * sizeof(float),
-              "the per-LOR values reuse the chunk's space");
+              "the per-LOR values reuse the rows' space");
 
 typedef float float2u __attribute__((ext_vector_type(2), aligned(4)));
 typedef float float4u __attribute__((ext_vector_type(4), aligned(8)));
@@ -181,19 +192,16 @@ typedef float float4u __attribute__((ext_vector_type(4), aligned(8)));
 typedef unsigned int uint2s __attribute__((ext_vector_type(2), aligned(8)));
 typedef unsigned int uint16s __attribute__((ext_vector_type(16), aligned(8)));
 
-// VEC: the replicates of a voxel are the sub-batch's (nbt = NB, aligned), so
-// that two planes are one load.
+// VEC: the replicates of a voxel are the sub-batch's (nbt = NB, aligned): one load.
 template <int MODE, int NB, bool VEC>
 __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
     const GeomView NIPET_CONST *gp, const float *__restrict__ img, float *__restrict__ sino,
     const int32_t *__restrict__ subs, const uint16_t *__restrict__ prompts,
     const float *__restrict__ rho, int rho_nb, Batch bt) {
   __shared__ __align__(16) double E[NB][FZ_NE];
-  __shared__ __align__(16) float D[NB][FZ_NE];
-  __shared__ double tot[NB][FZ_NG][128];
+  __shared__ double tot[NB][128];
   __shared__ double cend[NB][128];
   __shared__ float cmax[NB][2];
-  __shared__ int2 cl[MAX_SEG + FZ_CH];  // the bin's segments: (length, column)
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row = blockIdx.x;
@@ -208,83 +216,64 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
   int beg, nseg;
   const int first = seg_range_u(gp->off, bt.win, aw, beg, nseg);
   const SegRec NIPET_CONST *seg = (const SegRec NIPET_CONST *)(gp->seg + beg);
-  for (int i = tid; i < nseg + FZ_CH; i += FZ_THREADS)
-    cl[i] = make_int2(i < nseg ? __float_as_int(gp->seg[beg + i].len) : 0, gp->seg[beg + i].colz);
   // crossings of ring difference d: ev[ev_off(d) + w]
   const int nev = ev_off(dmax + 1);
   const uint2s NIPET_CONST *ev = (const uint2s NIPET_CONST *)(gp->ev + (size_t)aw * nev);
   // the bin's crossings on their way to L2 (a line per thread)
   float touch = 0.f;
   if (tid * 4 < nev) touch = __uint_as_float(gp->ev[(size_t)aw * nev + tid * 4].y);
-  if (tid < 64) {
+  // (finite everywhere: lanes past ring 63 read rows that are not staged yet)
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
-      E[b][FZ_CH * 128 + tid] = 0.0;
-      D[b][FZ_CH * 128 + tid] = 0.f;
-    }
-  }
+  for (int b = 0; b < NB; b++)
+    for (int i = tid; i < FZ_NE; i += FZ_THREADS) E[b][i] = 0.0;
 
-  // the wave's ring differences
-  const int ds[FZ_NS] = {63 - wv, 32 + wv, 31 - wv, wv};
+  // the crossing waves' ring differences, from dmax down in turns: slots 0 .. 2
+  // from 32 up (only rings r0 < 32 start a LOR), 3 .. 5 below; -1: none
+  const int cw = wv - FZ_SW, top = min(dmax, 31);
+  int ds[FZ_NS] = {dmax - cw, dmax - 2 * FZ_CW + 1 + cw, dmax - 2 * FZ_CW - cw,
+                   top - cw,  top - 2 * FZ_CW + 1 + cw,  top - 2 * FZ_CW - cw};
+#pragma unroll
+  for (int i = 0; i < FZ_NS; i++)
+    if (cw < 0 || ds[i] < (i < 3 ? 32 : 0)) ds[i] = -1;
   const bool mir = lane >= 32;  // lanes of the mirrors
   const int sg2 = mir ? -2 : 0;
-  double acc[FZ_NS][2][NB];  // ([0 .. 1][1] are not used)
-  float af[FZ_NS][2][NB];    // the a D terms apart, in float32
+  double acc[FZ_NS][2][NB];  // ([0 .. 2][1] are not used)
 #pragma unroll
   for (int i = 0; i < FZ_NS; i++)
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
-      acc[i][0][b] = acc[i][1][b] = 0.0;
-      af[i][0][b] = af[i][1][b] = 0.f;
-    }
+    for (int b = 0; b < NB; b++) acc[i][0][b] = acc[i][1][b] = 0.0;
 
-  // staging: group gr handles rows gr FZ_RPG .. of a chunk; its first wave the
-  // even planes p = 2 lane, its second the odd ones, each with plane p + 1
-  // (lane 63: plane 126 alone, and in the odd wave a plane 127 that is not used)
-  const int gr = wv >> 1, odd = wv & 1;
-  const int e0 = odd * 64 + lane;
-  const unsigned pl = min(2 * lane + odd, NZ - 1);
-  const bool even = nbt % 2 == 0 && b0 % 2 == 0 && (uintptr_t)img % 8 == 0;  // grid-uniform
-  float x0[FZ_RPG][NB], x1[FZ_RPG][NB];
-  // (Rows past the list have length 0 and some column of the image. A list's
-  // columns lie inside the field of view, never the image's last: plane 127 of
-  // one is plane 0 of the next.)
-  auto fetch = [&](int c) {
-    int64_t v0[FZ_RPG];
+  // staging: wave 0 has planes p = lane < 63, wave 1 planes 63 + lane, the next
+  // plane's value from the next lane (plane 127: 0). One register a row and
+  // replicate, so that a whole chunk is on its way.
+  const int pl = min(wv, 1) * 63 + lane;
+  const bool own = wv > 0 || lane < 63;
+  const int e0 = own ? (pl & 1) * 64 + (pl >> 1) : 127;  // (plane 127 is not used)
+  float x0[FZ_PF][NB];
+  // lane r: length (bits) of row r of the chunk that is staged, and of the next
+  // chunk and its columns, whose values are fetched meanwhile
+  int len = 0, len1, col1;
+  // (rows past the list have length 0 and some column of the image)
+  const char *im = (const char *)(img + b0);
+  const unsigned vb = 4 * (VEC ? NB : nbt);  // bytes of a voxel
+  auto fetch = [&](auto rc) {
+    constexpr int r = decltype(rc)::value;
+    // scalar base + 32-bit offset (an image has less than 4 GB)
+    const unsigned o = (unsigned)__builtin_amdgcn_readlane(col1, r) * vb + pl * vb;
+    if constexpr (VEC && NB == 2) {
+      const float2 t = *(const float2 *)(im + o);
+      x0[r][0] = t.x;
+      x0[r][NB - 1] = t.y;
+    } else {
 #pragma unroll
-    for (int r = 0; r < FZ_RPG; r++)
-      v0[r] = __builtin_amdgcn_readfirstlane(cl[c + gr * FZ_RPG + r].y);
-#pragma unroll
-    for (int r = 0; r < FZ_RPG; r++) {
-      if constexpr (VEC) {
-        if constexpr (NB == 1) {
-          const float2u t = *(const float2u *)((img + v0[r]) + pl);
-          x0[r][0] = t.x;
-          x1[r][0] = t.y;
-        } else {
-          const float4u t = *(const float4u *)((img + v0[r] * 2) + pl * 2);
-          x0[r][0] = t.x;
-          x0[r][NB - 1] = t.y;
-          x1[r][0] = t.z;
-          x1[r][NB - 1] = t.w;
-        }
-      } else {
-        const float *q = (img + v0[r] * nbt + b0) + (size_t)pl * nbt;
-        if (NB == 2 && even) {
-          const float2 t = *(const float2 *)q, u = *(const float2 *)(q + nbt);
-          x0[r][0] = t.x;
-          x0[r][NB - 1] = t.y;
-          x1[r][0] = u.x;
-          x1[r][NB - 1] = u.y;
-        } else {
-#pragma unroll
-          for (int b = 0; b < NB; b++) {
-            x0[r][b] = q[b];
-            x1[r][b] = q[nbt + b];
-          }
-        }
-      }
+      for (int b = 0; b < NB; b++) x0[r][b] = *(const float *)(im + o + 4 * b);
     }
+  };
+  auto records = [&](int j0) {  // the chunk from segment j0 on
+    const int j = j0 + min(lane, FZ_CH - 1);
+    const int2 t = *(const int2 *)&gp->seg[beg + j].len;
+    len1 = j < nseg ? t.x : 0;
+    col1 = t.y;
   };
   double carry[NB];
   float cmx[NB];
@@ -293,123 +282,70 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
     carry[b] = 0.0;
     cmx[b] = 0.f;
   }
-  int wn[FZ_NS] = {0, 0, 0, 0};  // slot i: the next crossing's plane offset
-  __syncthreads();
-  if (nseg > 0) {
-    fetch(0);
-    const double t0 = seg[0].s * (2.0 / gp->atn[aw]);
-    // plane offset at the start, rounded down on a tie, then past the crossings
-    // of earlier segments
-    unsigned first_ev[FZ_NS];
+  // rows first + c + 1 .. first + c + FZ_CH, each read again FZ_PF segments on
+  auto stage = [&](int c) {
+    static_for<FZ_PF>([&](auto rc) {
+      constexpr int r = decltype(rc)::value;
+      const int slot = (first + c + r + 1) & (FZ_RING - 1);
+      const float L = __int_as_float(__builtin_amdgcn_readlane(len, r));
 #pragma unroll
-    for (int i = 0; i < FZ_NS; i++) {
-      const int d = max(min(ds[i], dmax), 0);
-      wn[i] = max(__builtin_amdgcn_readfirstlane((int)floor(fma((double)d, t0, 0.5 - 1e-9))), 0);
-      first_ev[i] = d > 0 ? ev[ev_off(d) + wn[i]].x : ~0u;
-    }
+      for (int b = 0; b < NB; b++) {
+        const float x1 = __int_as_float(__builtin_amdgcn_update_dpp(
+            0, __float_as_int(x0[r][b]), 0x130 /* wave_shl:1 */, 0xf, 0xf, true));
+        carry[b] = fma((double)L, (double)x0[r][b] - (double)x1, carry[b]);
+        E[b][slot * 128 + e0] = carry[b];
+        if (slot == 0) E[b][FZ_RING * 128 + e0] = carry[b];
+      }
+      fetch(rc);
+    });
+    len = len1;
+    records(c + 2 * FZ_CH);
 #pragma unroll
-    for (int i = 0; i < FZ_NS; i++)
-      while ((int)(first_ev[i] >> 10) < first)
-        first_ev[i] = ev[ev_off(min(ds[i], dmax)) + ++wn[i]].x;
-  }
+    for (int b = 0; b < NB; b++) cmx[b] = fmaxf(cmx[b], fabsf((float)carry[b]));
+  };
+  int wn[FZ_NS] = {0, 0, 0, 0, 0, 0};  // slot i: the next crossing's plane offset
   // the next eight crossings of slot i (a list ends in eight past any segment)
   auto next8 = [&](int i, int w) {
-    return *(const uint16s NIPET_CONST *)(ev + ev_off(max(min(ds[i], dmax), 1)) + w);
+    return *(const uint16s NIPET_CONST *)(ev + ev_off(max(ds[i], 1)) + w);
   };
-  for (int c = 0; c < nseg; c += FZ_CH) {
-    float len[FZ_RPG];
-#pragma unroll
-    for (int r = 0; r < FZ_RPG; r++) len[r] = __int_as_float(cl[c + gr * FZ_RPG + r].x);
-    double dd[FZ_RPG][NB];
-    {
-      double t[NB];
-#pragma unroll
-      for (int b = 0; b < NB; b++) t[b] = 0.0;
-#pragma unroll
-      for (int r = 0; r < FZ_RPG; r++) {
-        const double L = (double)len[r];
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-          dd[r][b] = (double)x0[r][b] - (double)(lane < 63 ? x1[r][b] : 0.f);
-          t[b] = fma(L, dd[r][b], t[b]);
-        }
-      }
-#pragma unroll
-      for (int b = 0; b < NB; b++) tot[b][gr][e0] = t[b];
-    }
-    __syncthreads();  // totals written; the previous chunk's crossings done
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-      double base = carry[b], sum = carry[b];
-      static_for<FZ_NG / 4>([&](auto qc) {  // four in flight (registers)
-        constexpr int q0 = decltype(qc)::value * 4;
-        double t[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) t[q] = tot[b][q0 + q][e0];
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          if (q0 + q == gr) {  // wave-uniform
-            base = sum;
-            asm volatile("; the group's first row");
-          }
-          sum += t[q];
-        }
-      });
-      carry[b] = sum;
-      cmx[b] = fmaxf(cmx[b], fabsf((float)sum));
-#pragma unroll
-      for (int r = 0; r < FZ_RPG; r++) {
-        const int j = gr * FZ_RPG + r;
-        E[b][j * 128 + e0] = base;
-        D[b][j * 128 + e0] = (float)dd[r][b];
-        base = fma((double)len[r], dd[r][b], base);
-      }
-    }
-    __syncthreads();
-    if (c + FZ_CH < nseg) fetch(c + FZ_CH);
-    if (c == 0) asm volatile("" ::"v"(touch));
-
-    const int jb = (first + c) << 10;
+  auto cross = [&](int c) {
     // crossings in segments below je belong to this chunk (past the list: none)
     const unsigned je = (unsigned)(first + min(c + FZ_CH, nseg)) << 10;
     uint16s nx = next8(0, wn[0]);
     static_for<FZ_NS>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
-      constexpr int NK = i >= 2 ? 2 : 1;  // rings 32 .. 63 start LORs too
+      constexpr int NK = i >= 3 ? 2 : 1;  // rings 32 .. 63 start LORs too
       const int d = ds[i];
       uint16s cu = nx;
       if constexpr (i + 1 < FZ_NS) nx = next8(i + 1, wn[i + 1]);
-      if (d <= 0 || d > dmax) return;
-      const int lb = 8 * (lane & 31) + (mir ? 512 + 8 * (d - 1) : 0) - jb;
+      if (d <= 0) return;
+      const int lb = 8 * (lane & 31) + (mir ? 512 + 8 * (d - 1) : 0);
       // N crossings cu[2 q0 ..]: all reads first
       auto some = [&](auto nc, auto qc) {
         constexpr int N = decltype(nc)::value, q0 = decltype(qc)::value;
-        double ev_[N][NK][NB];
-        float dv[N][NK][NB];
+        double ea[N][NK][NB], eb[N][NK][NB];
 #pragma unroll
         for (int n = 0; n < N; n++) {
           const unsigned wd = cu[2 * (q0 + n)];
-          const int va = (int)wd + (lb + sg2 * (int)(wd & 1023));
+          const int va = (int)(wd & (FZ_RING * 1024 - 1)) + (lb + sg2 * (int)(wd & 1023));
           const char *pe = (const char *)&E[0][0] + va;
-          const char *pd = (const char *)&D[0][0] + (va >> 1);
 #pragma unroll
           for (int b = 0; b < NB; b++)
 #pragma unroll
             for (int k = 0; k < NK; k++) {
-              ev_[n][k][b] = *(const double *)(pe + b * FZ_NE * 8 + 256 * k);
-              dv[n][k][b] = *(const float *)(pd + b * FZ_NE * 4 + 128 * k);
+              ea[n][k][b] = *(const double *)(pe + b * FZ_NE * 8 + 256 * k);
+              eb[n][k][b] = *(const double *)(pe + b * FZ_NE * 8 + 256 * k + 1024);
             }
         }
 #pragma unroll
-        for (int n = 0; n < N; n++)
+        for (int n = 0; n < N; n++) {
+          const double f = __hiloint2double(cu[2 * (q0 + n) + 1], cu[2 * (q0 + n)]);
 #pragma unroll
           for (int b = 0; b < NB; b++)
 #pragma unroll
-            for (int k = 0; k < NK; k++) {
-              acc[i][k][b] += ev_[n][k][b];
-              af[i][k][b] = fmaf(__uint_as_float(cu[2 * (q0 + n) + 1]), dv[n][k][b], af[i][k][b]);
-            }
+            for (int k = 0; k < NK; k++)
+              acc[i][k][b] = fma(f, eb[n][k][b] - ea[n][k][b], acc[i][k][b] + ea[n][k][b]);
+        }
       };
       using std::integral_constant;
       constexpr int N = NK * NB >= 2 ? 2 : 4;  // crossings read at once (registers)
@@ -420,13 +356,13 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
         int done = 0;
         static_for<8 / N>([&](auto qc) {
           constexpr int q = decltype(qc)::value * N;
-          if (done == q && cu[2 * (q + N - 1)] < je) {
+          if (done == q && (cu[2 * (q + N - 1)] & EV_PLACE) < je) {
             some(nc, integral_constant<int, q>{});
             done = q + N;
           } else if (done == q) {
             static_for<N - 1>([&](auto rc) {
               constexpr int r = decltype(rc)::value;
-              if (done == q + r && cu[2 * (q + r)] < je) {
+              if (done == q + r && (cu[2 * (q + r)] & EV_PLACE) < je) {
                 some(integral_constant<int, 1>{}, integral_constant<int, q + r>{});
                 done = q + r + 1;
               }
@@ -440,37 +376,76 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
       } while (full);
       wn[i] = w;
     });
+  };
+  // a chunk is staged while the one before it is crossed: as many barriers on
+  // both sides (apart, so that neither side's registers burden the other)
+  if (wv < FZ_SW) {
+    if (nseg > 0) {
+      records(0);
+      static_for<FZ_PF>([&](auto rc) { fetch(rc); });
+      len = len1;
+      records(FZ_CH);
+    }
+    __syncthreads();  // the rows cleared
+    for (int c = 0; c < nseg; c += FZ_CH) {
+      stage(c);
+      __syncthreads();
+    }
+  } else {
+    if (nseg > 0) {
+      const double t0 = seg[0].s * (2.0 / gp->atn[aw]);
+      // plane offset at the start, rounded down on a tie, then past the crossings
+      // of earlier segments
+      unsigned first_ev[FZ_NS];
+#pragma unroll
+      for (int i = 0; i < FZ_NS; i++) {
+        const int d = max(ds[i], 0);
+        wn[i] = max(__builtin_amdgcn_readfirstlane((int)floor(fma((double)d, t0, 0.5 - 1e-9))), 0);
+        first_ev[i] = d > 0 ? ev[ev_off(d) + wn[i]].x : ~0u;
+      }
+#pragma unroll
+      for (int i = 0; i < FZ_NS; i++)
+        while ((int)((first_ev[i] & EV_PLACE) >> 10) < first)
+          first_ev[i] = ev[ev_off(ds[i]) + ++wn[i]].x;
+    }
+    __syncthreads();
+    for (int c = 0; c < nseg; c += FZ_CH) {
+      __syncthreads();  // the chunk staged
+      cross(c);
+    }
   }
+  __syncthreads();  // the last chunk's crossings done (the rows' space is used again)
+  asm volatile("" ::"v"(touch));
 
   // C_p(t_end) = sum of the total differences from plane p up, and the largest
   // magnitude of the prefix sums
-  __syncthreads();  // the last chunk's crossings done
   bool bad = false;
-  if (gr == 0) {
+  if (wv < FZ_SW) {
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-      bad |= !isfinite(carry[b]);
-      float m = cmx[b];
+      bad |= own && !isfinite(carry[b]);
+      float m = own ? cmx[b] : 0.f;
       for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-      if (lane == 0) cmax[b][odd] = m;
-      tot[b][0][2 * lane + odd] = (odd && lane == 63) ? 0.0 : carry[b];
+      if (lane == 0) cmax[b][wv] = m;
+      if (own) tot[b][pl] = carry[b];
+      if (wv == 0 && lane == 63) tot[b][127] = 0.0;
     }
   }
   const bool slow = __syncthreads_or(bad);
-  if (gr == 0) {  // wave 0: planes 0 .. 63; wave 1: 64 .. 127; each a suffix sum
+  if (wv < FZ_SW) {  // wave 0: planes 0 .. 63; wave 1: 64 .. 127; each a suffix sum
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-      double v = tot[b][0][odd * 64 + lane];
+      double v = tot[b][wv * 64 + lane];
       for (int o = 1; o < 64; o <<= 1) {
         const double u = __shfl_down(v, o);
         if (lane + o < 64) v += u;
       }
-      if (odd == 0) {  // + all of planes 64 .. 127
-        double h = tot[b][0][64 + lane];
+      if (wv == 0) {  // + all of planes 64 .. 127
+        double h = tot[b][64 + lane];
         for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
         v += h;
       }
-      const int p = odd * 64 + lane;
+      const int p = wv * 64 + lane;
       cend[b][(p & 1) * 64 + (p >> 1)] = v;
     }
   }
@@ -486,10 +461,10 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
     static_for<FZ_NS>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
       const int d = ds[i];
-      if (d > dmax) return;
+      if (d < 0) return;
       const float sf = lor_sfac(2.f * d, gp->vox_z, atn);
 #pragma unroll
-      for (int k = 0; k < (i < 2 ? 1 : 2); k++) {
+      for (int k = 0; k < (i < 3 ? 1 : 2); k++) {
         const int r0 = (lane & 31) + 32 * k;
         const int li = r0 + d <= 63 ? gp->dr_li[d * 64 + r0] : -1;
         if (li < 0 || (mir && d == 0)) continue;
@@ -514,7 +489,7 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
           }
         } else {
           const int pz = (mir ? 2 * d - wn[i] : wn[i]) + 2 * r0;
-          const double x = acc[i][k][b] + (double)af[i][k][b];
+          const double x = acc[i][k][b];
           v = cend[b][(pz & 1) * 64 + (pz >> 1)] + (mir ? -x : x);
           if (fabs(v) <= snap) v = 0.0;
         }
