@@ -601,11 +601,11 @@ static int geom_build(const NipetGeomDesc *d, NipetGeom *g) {
   k_tx_lists<<<nb, 256>>>(d_crs, d_s2c, d->naw, (double)d->vox_xy, (double)d->tfov2, NZ, g->off,
                           nullptr, g->seg, nullptr, g->lmax, d_err);
   NIPET_HIP(hipGetLastError());
-  if (g->dmax > 0) {  // eight crossings are read at a time
+  {  // eight crossings are read at a time, also where there are none (dmax 0)
     const size_t ne = ev_off(g->dmax + 1);
     NIPET_HIP(hipMalloc(&g->ev, (d->naw * ne + 8) * sizeof(uint2)));
     NIPET_HIP(hipMemset(g->ev + d->naw * ne, 0xff, 8 * sizeof(uint2)));
-    k_events<<<d->naw, 256>>>(g->off, g->seg, g->atn, g->dmax, g->ev);
+    if (ne > 0) k_events<<<d->naw, 256>>>(g->off, g->seg, g->atn, g->dmax, g->ev);
     NIPET_HIP(hipGetLastError());
   }
   NIPET_HIP(hipDeviceSynchronize());

@@ -245,3 +245,24 @@ def test_staged_equals_atomics(torch, lib, params, n, per, nb):
         for b in range(nb):
             one = back(torch, lib, geom, y[..., b].contiguous(), rows, n)
             assert float((got[..., b] - one).abs().max()) < 1e-6 * float(one.max())
+
+
+@pytest.mark.parametrize('dmax', [0, 1, 7])
+def test_few_ring_differences(torch, lib, params, dmax):
+    """Michelograms of the first ring differences only (none of them crosses a
+    plane at dmax 0): the projections by segments, and the adjoint of them."""
+    from nipet_amd.geom import DeviceGeom
+    ax = params['axLUT']
+    sel = np.abs(ax['li2rng'][:, 0] - ax['li2rng'][:, 1]) < (dmax + 0.5) * params['Cnt']['AXR']
+    few = dict(params, axLUT=dict(ax, **{k: ax[k][sel] for k in ('li2rng', 'li2sn', 'li2nos')}))
+    geom, rows = DeviceGeom(few, torch.cuda.current_device()), rows_of(torch, 40, 31)
+    g = torch.Generator(device='cuda').manual_seed(6)
+    img = torch.rand((320, 320, 127), generator=g, device='cuda')
+    out = [torch.full((len(rows), geom.nsn), 9.0, device='cuda') for _ in range(2)]
+    for o, name in zip(out, ('nipet_fprj', 'nipet_fprj_seg')):
+        lib.check(getattr(lib.lib(), name)(geom.handle, lib.ptr(o), lib.ptr(img), lib.ptr(rows),
+                                           len(rows), 0, lib.stream_handle()), name)
+    assert float((out[0] - out[1]).abs().max()) < BAR * float(out[1].max())
+    y = torch.rand((len(rows), geom.nsn), generator=g, device='cuda')
+    dot = float((back(torch, lib, geom, y, rows).double() * img).sum())
+    assert abs(dot / float((out[0].double() * y).sum()) - 1) < 1e-6
