@@ -53,7 +53,7 @@ def autotune(state, widths=(4, 2, 1), repeats=2, probe=4):
     ``state`` (an ``OsemBatch``) over a probe batch of min(nb, ``probe``)
     replicates, and keep the fastest shape per kernel: the FP sub-batch width,
     and the BP sub-batch width together with its run length (segments per
-    wave run: each width has two compiled run lengths). Results are cached
+    wave run, kept as a setting: the kernel gives every wave one run). Results are cached
     per (geometry, subset size) for the process. Returns {'fprj': w, 'bprj': w,
     'bprj_run': {w: segments}, 'ms': {(kernel, w[, run]): ms per image}}."""
     import ctypes as ct
