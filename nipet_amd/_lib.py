@@ -154,27 +154,39 @@ def stream_handle(device=None):
 
 def bprj_scratch(geom, nprj, nb=1):
     """Device buffer for staged back projections of ``nprj`` bins of ``nb``
-    images (``nipet_bprj_scratch``), or None where none is used."""
+    images (``nipet_bprj_scratch``), or None where none is used or the device has
+    no room for it (the projections then add to the image directly)."""
     import torch
     n = lib().nipet_bprj_scratch(geom.handle, int(nprj), int(nb))
-    return torch.empty(n, dtype=torch.uint8, device='cuda') if n else None
+    try:
+        return torch.empty(n, dtype=torch.uint8, device='cuda') if n else None
+    except torch.OutOfMemoryError:
+        return None
+
+
+_scratch = threading.local()
 
 
 class scratch:
     """Context manager: this thread's back projections use the device buffer
-    ``buf`` (``nipet_scratch_set``; None: none). The buffer belongs to the
-    stream the calls run on."""
+    ``buf`` (``nipet_scratch_set``; None: none), afterwards the one before. The
+    buffer belongs to the stream the calls run on."""
 
     def __init__(self, buf):
         self.buf = buf
 
-    def __enter__(self):
-        b = self.buf
-        check(lib().nipet_scratch_set(ptr(b), 0 if b is None else b.numel()),
+    @staticmethod
+    def _set(buf):
+        check(lib().nipet_scratch_set(ptr(buf), 0 if buf is None else buf.numel()),
               'nipet_scratch_set')
+        _scratch.buf = buf
+
+    def __enter__(self):
+        self.before = getattr(_scratch, 'buf', None)
+        self._set(self.buf)
 
     def __exit__(self, *exc):
-        check(lib().nipet_scratch_set(None, 0), 'nipet_scratch_set')
+        self._set(self.before)
         return False
 
 

@@ -266,3 +266,22 @@ def test_few_ring_differences(torch, lib, params, dmax):
     y = torch.rand((len(rows), geom.nsn), generator=g, device='cuda')
     dot = float((back(torch, lib, geom, y, rows).double() * img).sum())
     assert abs(dot / float((out[0].double() * y).sum()) - 1) < 1e-6
+
+
+def test_scratch_nests(torch, lib, params):
+    """Leaving an inner scratch context gives the outer one back: staged sums
+    (the same bits) and not atomics; without room there is no buffer."""
+    from nipet_amd.geom import get_geom
+    geom, rows = get_geom(params), rows_of(torch, 2000, 41)
+    y = torch.rand((len(rows), geom.nsn), device='cuda')
+    outer = lib.bprj_scratch(geom, len(rows))
+    imgs = [torch.zeros((320, 320, 127), device='cuda') for _ in range(2)]
+    with lib.scratch(outer):
+        for im in imgs:
+            with lib.scratch(None):
+                pass
+            outer.fill_(255)
+            lib.check(lib.lib().nipet_bprj_b(geom.handle, lib.ptr(im), lib.ptr(y), lib.ptr(rows),
+                                             len(rows), 1, lib.stream_handle()), 'nipet_bprj_b')
+            assert not bool((outer == 255).all())  # the rows went there
+    assert torch.equal(*imgs)
