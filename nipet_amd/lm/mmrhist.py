@@ -147,10 +147,14 @@ class LmHistogram:
                                               self._on_stream()), 'nipet_lm_finish')
 
     def _on_stream(self):
-        """Handle of the current stream, which the session's memory outlives."""
+        """Handle of the current stream. What the kernels use was allocated on
+        the session's first stream: on another one it is recorded, so that its
+        memory is not given out again before that stream has done with it (a
+        session that is dropped waits for nothing)."""
         st = _torch().cuda.current_stream()
         if st != self._stream:
-            self._mem.record_stream(st)
+            for t in (self._mem, *self.out.values()):
+                t.record_stream(st)
         return st.cuda_stream
 
     def status(self):

@@ -255,7 +255,7 @@ def _remgaps_b(h, scanner_params, nrep, r0, nb, out=None, out_b0=0):
         raise ValueError(f'prompts output must be a contiguous ({naw}, {nsn}, n) tensor')
     _lib.check(_lib.lib().nipet_remgaps_u16b(_lib.ptr(out), _lib.ptr(h.out['psino']),
                                              _lib.ptr(ali), naw, nsn, 86688, nrep, r0, nb,
-                                             out.shape[2], out_b0, _lib.stream_handle()),
+                                             out.shape[2], out_b0, h._on_stream()),
                'nipet_remgaps_u16b')
     return out
 
