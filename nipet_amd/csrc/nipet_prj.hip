@@ -927,9 +927,13 @@ __global__ __launch_bounds__(256) void k_seg_window(GeomView g, const uint8_t *_
 // instructions in every segment: 1.24 ms a subset of 4,894 bins.)
 //  - What enters leaves again in the same pairs (va, vb), so S_p in float64
 //    returns to its former value to 1e-16 of the bin's largest value, and
-//    sums below BP_SNAP of that are set to 0: a plane that no LOR is on gets
+//    S_p below BP_SNAP of that are set to 0: a plane that no LOR is on gets
 //    nothing. The segment's own sum is float64 too (full-rate FP64): a short
 //    piece of a segment is a difference here.
+//  - A bin with values below BP_FAINT of its largest (zeros aside) may have S_p
+//    that small beside the rounding of the large ones. There a wave that meets
+//    one sums its run again, segment by segment, from the terms themselves
+//    (without a row to overwrite, every run of such a bin is).
 //  - S and the segment's sum carry the sign (-1)^p, so that a crossing adds (w
 //    even) or subtracts (w odd) one T for all lanes: no per-lane sign.
 //  - va / vb (times the 3D length factor of d) sit in LDS, row d at 65 d with
@@ -942,7 +946,8 @@ __global__ __launch_bounds__(256) void k_seg_window(GeomView g, const uint8_t *_
 //    ten of them and two LDS reads. Finding the crossings with lane d on ring
 //    difference d and a ballot per segment, and v_readlane for each: 0.57 ms.
 //  - Non-finite sinogram values would stay in S after their LOR has left the
-//    plane: such a bin is summed segment by segment.
+//    plane, and so would the overflow of huge ones: a bin with values from
+//    BP_HUGE up is summed segment by segment.
 //  - Output: with STAGED every segment's plane sums go to the segment's own row
 //    of a scratch buffer (512 bytes an image) and k_bp_gather adds the rows of
 //    each voxel column, else float atomics to the image.
@@ -952,7 +957,7 @@ template <int NB>
 constexpr int bp_threads() {
   return 512 * NB;
 }
-constexpr float BP_SNAP = 0x1p-47f;
+constexpr float BP_SNAP = 0x1p-45f, BP_FAINT = 0x1p-21f, BP_HUGE = 0x1p120f;
 
 //
 // img: the image [voxel][nbt] (atomics, zeroed before), or with STAGED the
@@ -966,7 +971,9 @@ __global__ __launch_bounds__(bp_threads<NB>(), 8) void k_bprj(
   // vb, an entry that is not used (an odd crossing's va look-up is at lane - 1)
   // and va; first the sinogram row and a zero are staged there
   __shared__ __align__(16) float tab[(2 * BP_TN + 1) * NB];
-  __shared__ int vmax;  // largest magnitude in tab (its bits)
+  // per image: largest magnitude in the row, and smallest other than 0, minus 1
+  // (bits without the sign)
+  __shared__ unsigned vtop[NB], vlow[NB];
   float *srow = tab;
   static_assert(sizeof(tab) >= 4096 * NB * sizeof(float), "a row of 4095 sinograms");
   const int tid = threadIdx.x, lane = tid & 63;
@@ -982,26 +989,35 @@ __global__ __launch_bounds__(bp_threads<NB>(), 8) void k_bprj(
 
   // sinogram rows in subset order, or (by_bin) the full [naw][nsn] sinogram
   // read at the bin's own row; sino2: the second of two images, by bin
-  bool bad = false;
-  if (NB == 2 && sino2) {
-    const float *in = sino + (size_t)row * nsn, *in2 = sino2 + (size_t)aw * nsn;
-    for (int i = tid; i <= nsn; i += THR) {
-      const float x = i < nsn ? in[i] : 0.f, y = i < nsn ? in2[i] : 0.f;
-      bad |= !isfinite(x) || !isfinite(y);
-      srow[i * NB] = x;
-      srow[i * NB + NB - 1] = y;
-    }
-  } else {
-    const float *in = sino + (size_t)(by_bin ? aw : row) * nsn * nbt + b0;
-    for (int i = tid; i < (nsn + 1) * NB; i += THR) {
-      const int s = i / NB, b = i - s * NB;
-      const float x = s < nsn ? in[(size_t)s * nbt + b] : 0.f;
-      bad |= !isfinite(x);
-      srow[i] = x;
+  unsigned top = 0, low = ~0u;  // of the thread's image
+  {
+    const int b = tid % NB;
+    const bool two = NB == 2 && sino2;
+    const float *in = sino + (size_t)(by_bin ? aw : row) * nsn * (two ? 1 : nbt);
+    in += two ? 0 : b0 + b;
+    if (two && b) in = sino2 + (size_t)aw * nsn;
+    const int step = two ? 1 : nbt;
+    for (int k = tid / NB; k <= nsn; k += THR / NB) {
+      const float x = k < nsn ? in[(size_t)k * step] : 0.f;
+      const unsigned u = __float_as_uint(x) << 1;
+      top = max(top, u);
+      low = min(low, u - 1u);
+      srow[k * NB + b] = x;
     }
   }
-  if (tid == 0) vmax = 0;
-  const bool slow = __syncthreads_or(bad);
+  if (tid < NB) {
+    vtop[tid] = 0;
+    vlow[tid] = ~0u;
+  }
+  __syncthreads();
+  for (int o = 32; o >= NB; o >>= 1) {
+    top = max(top, (unsigned)__shfl_xor((int)top, o));
+    low = min(low, (unsigned)__shfl_xor((int)low, o));
+  }
+  if (lane < NB) {
+    atomicMax(&vtop[lane], top);
+    atomicMin(&vlow[lane], low);
+  }
   float xa[IT][NB], xb[IT][NB];
 #pragma unroll
   for (int k = 0; k < IT; k++) {
@@ -1013,7 +1029,6 @@ __global__ __launch_bounds__(bp_threads<NB>(), 8) void k_bprj(
     }
   }
   __syncthreads();
-  float top = 0.f;
 #pragma unroll
   for (int k = 0; k < IT; k++) {
     const int i = tid + k * THR;
@@ -1021,16 +1036,23 @@ __global__ __launch_bounds__(bp_threads<NB>(), 8) void k_bprj(
     const float sf = lor_sfac(2.f * (float)(i / 65), gp->vox_z, atn);  // (padding is 0)
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-      const float x = xa[k][b] * sf, y = xb[k][b] * sf;
-      tab[i * NB + b] = y;
-      tab[(BP_TN + 1 + i) * NB + b] = x;
-      top = fmaxf(top, fmaxf(fabsf(x), fabsf(y)));
+      tab[i * NB + b] = xb[k][b] * sf;
+      tab[(BP_TN + 1 + i) * NB + b] = xa[k][b] * sf;
     }
   }
-  for (int o = 32; o > 0; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
-  if (lane == 0) atomicMax(&vmax, __float_as_int(top));
   __syncthreads();
-  const float snap = slow ? 0.f : BP_SNAP * __int_as_float(vmax);
+  bool huge = false, faint = false;
+  float snap[NB];  // sums that do not count: of empty planes, or (faint) to be summed again
+#pragma unroll
+  for (int b = 0; b < NB; b++) {
+    const unsigned ut = __builtin_amdgcn_readfirstlane(vtop[b]),
+                   ul = __builtin_amdgcn_readfirstlane(vlow[b]) + 1u;
+    const float t = __uint_as_float(ut >> 1), l = __uint_as_float(ul >> 1);
+    huge |= !(t < BP_HUGE);
+    const bool f = l < BP_FAINT * t;
+    faint |= f;
+    snap[b] = (f ? BP_FAINT : BP_SNAP) * t;
+  }
 
   // lane d: crossings of ring difference d
   const bool on = lane >= 1 && lane <= dmax;
@@ -1057,19 +1079,22 @@ __global__ __launch_bounds__(bp_threads<NB>(), 8) void k_bprj(
   double s = seg[j0].s;
   int w = plane_offset(m, s);
 
-  // the sums of segment j0, j0 + 1, .. without their signs, to the segment's row
-  // or to the image
+  // the sums of segment j0, j0 + 1, .. (length len) without their signs, to the
+  // segment's row or to the image
   float *q = nullptr;
   if constexpr (STAGED)
     q = img + ((size_t)blockIdx.x * gp->maxseg + first + j0) * (128 * NB) + lane * 2 * NB;
-  auto put = [&](int colz, const double (&acc)[2][NB]) {
+  unsigned long long small[2] = {0, 0};  // lanes whose sums were set to 0
+  auto put = [&](int colz, float len, const double (&acc)[2][NB]) {
     float v[2 * NB];
 #pragma unroll
     for (int k = 0; k < 2; k++)
 #pragma unroll
       for (int b = 0; b < NB; b++) {
         v[k * NB + b] = (float)(k ? acc[k][b] : -acc[k][b]);
-        if (fabsf(v[k * NB + b]) <= snap) v[k * NB + b] = 0.f;
+        const bool z = fabsf(v[k * NB + b]) <= snap[b] * len;
+        if constexpr (STAGED) small[k] |= __builtin_amdgcn_ballot_w64(z);
+        if (z) v[k * NB + b] = 0.f;
       }
     if constexpr (STAGED) {
       stv<2 * NB>(q, v);
@@ -1088,47 +1113,13 @@ __global__ __launch_bounds__(bp_threads<NB>(), 8) void k_bprj(
     }
   };
 
-  double acc[2][NB];
-  if (slow) {
-    for (int j = j0; j < j1; j++) {
-      const double s1 = j + 1 < nseg ? seg[j + 1].s : s + (double)seg[j].len;
-      const int wn = plane_offset(m, s1);
-#pragma unroll
-      for (int b = 0; b < NB; b++) acc[0][b] = acc[1][b] = 0.0;
-      for (int d = 0; d <= dmax; d++) {
-        int wc = __builtin_amdgcn_readlane(w, d);
-        const int we = __builtin_amdgcn_readlane(wn, d);
-        double pos = s;
-        for (; wc <= we; wc++) {  // pieces of the segment on offset wc
-          const double end = wc < we ? fmin(((double)wc + 0.5) * atn / (2.0 * d), s1) : s1;
-          const int k = wc & 1, x = 4 * bp_entry(d, wc);
-          float T[2][NB];
-          lookup(x, 516 * d - x, T);
-          if (end > pos) {  // (signs as in the walk below)
-#pragma unroll
-            for (int b = 0; b < NB; b++) {
-              if (!k && T[0][b] != 0.f) acc[0][b] -= (end - pos) * (double)T[0][b];
-              if (k && T[1][b] != 0.f) acc[1][b] += (end - pos) * (double)T[1][b];
-            }
-          }
-          pos = end > pos ? end : pos;
-        }
-      }
-      put(seg[j].colz, acc);
-      w = wn;
-      s = s1;
-    }
-    return;
-  }
-
-  double S[2][NB];
-#pragma unroll
-  for (int b = 0; b < NB; b++) S[0][b] = S[1][b] = 0.0;
-  {
+  // sum of the LORs of ring differences ds on plane offset w
+  auto standing = [&](unsigned long long ds, double (&S)[2][NB]) {
     // LORs of d are on planes of w's parity
-    unsigned long long odd = __builtin_amdgcn_ballot_w64(w & 1),
-                       even = ~odd & (~0ull >> (63 - dmax));
+    unsigned long long odd = __builtin_amdgcn_ballot_w64(w & 1) & ds, even = ~odd & ds;
     const int x_l = 4 * bp_entry(lane, w);
+#pragma unroll
+    for (int b = 0; b < NB; b++) S[0][b] = S[1][b] = 0.0;
 #pragma unroll 2
     for (; even; even &= even - 1) {
       const int d = __builtin_ctzll(even), x = __builtin_amdgcn_readlane(x_l, d);
@@ -1145,7 +1136,54 @@ __global__ __launch_bounds__(bp_threads<NB>(), 8) void k_bprj(
 #pragma unroll
       for (int b = 0; b < NB; b++) S[1][b] += (double)T[1][b];
     }
+  };
+  const unsigned long long all = ~0ull >> (63 - dmax);
+
+  double acc[2][NB];
+  // the run segment by segment, each sum from its own terms
+  auto by_segment = [&]() {
+    const double inv = on ? atn / (2.0 * lane) : 0.0;
+    for (int j = j0; j < j1; j++) {
+      const double s1 = j + 1 < nseg ? seg[j + 1].s : s + (double)seg[j].len;
+      const int wn = plane_offset(m, s1);
+      unsigned long long hit = __builtin_amdgcn_ballot_w64(w < wn);
+      double S[2][NB];
+      standing(all & ~hit, S);
+#pragma unroll
+      for (int k = 0; k < 2; k++)
+#pragma unroll
+        for (int b = 0; b < NB; b++) acc[k][b] = s1 > s ? (s1 - s) * S[k][b] : 0.0;
+      for (; hit; hit &= hit - 1) {  // pieces of the ring differences that cross
+        const int d = __builtin_ctzll(hit), we = __builtin_amdgcn_readlane(wn, d);
+        const double step = rdlane(inv, d);
+        double pos = s;
+        for (int wc = __builtin_amdgcn_readlane(w, d); wc <= we; wc++) {
+          const double end = wc < we ? fmin(((double)wc + 0.5) * step, s1) : s1;
+          const int x = 4 * bp_entry(d, wc);
+          float T[2][NB];
+          lookup(x, 516 * d - x, T);
+          if (end > pos) {  // (signs as in the walk below)
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+              if (wc & 1) acc[1][b] += (end - pos) * (double)T[1][b];
+              else acc[0][b] -= (end - pos) * (double)T[0][b];
+            }
+            pos = end;
+          }
+        }
+      }
+      put(seg[j].colz, 0.f, acc);
+      w = wn;
+      s = s1;
+    }
+  };
+  if (huge || (faint && !STAGED)) {
+    by_segment();
+    return;
   }
+
+  double S[2][NB];
+  standing(all, S);
   // lane i: length and column of segment jb + i
   double Ll;
   int Cl = 0, jb;
@@ -1158,11 +1196,11 @@ __global__ __launch_bounds__(bp_threads<NB>(), 8) void k_bprj(
   };
   lengths(j0);
   int j = j0;
-  const double L0 = rdlane(Ll, 0);
+  double L = rdlane(Ll, 0);
 #pragma unroll
   for (int k = 0; k < 2; k++)
 #pragma unroll
-    for (int b = 0; b < NB; b++) acc[k][b] = L0 * S[k][b];
+    for (int b = 0; b < NB; b++) acc[k][b] = L * S[k][b];
   const uint2s NIPET_CONST *ev =
       (const uint2s NIPET_CONST *)(gp->bp_ev + ((const uint32_t NIPET_CONST *)gp->bp_off)[beg + j0]);
   uint32_t live = 1;  // 0 when the run is done (the rest of its last eight is not)
@@ -1186,9 +1224,9 @@ __global__ __launch_bounds__(bp_threads<NB>(), 8) void k_bprj(
           S[k][b] = fma(sg, (double)T[k][b], S[k][b]);
         }
       if (lo & live) {
-        put(__builtin_amdgcn_readlane(Cl, j - jb), acc);
+        put(__builtin_amdgcn_readlane(Cl, j - jb), (float)L, acc);
         live = __builtin_amdgcn_readfirstlane(++j < j1);
-        const double L = rdlane(Ll, j - jb);
+        L = rdlane(Ll, j - jb);
 #pragma unroll
         for (int k = 0; k < 2; k++)
 #pragma unroll
@@ -1203,6 +1241,11 @@ __global__ __launch_bounds__(bp_threads<NB>(), 8) void k_bprj(
     cur = *(const uint16s NIPET_CONST *)(ev + 16);
     eight(nxt);
     if (!live) break;
+  }
+  // (lane 63 has no plane 127)
+  if (STAGED && faint && (small[0] | (small[1] & (~0ull >> 1)))) {
+    q -= (size_t)(j1 - j0) * (128 * NB);
+    by_segment();
   }
 }
 
