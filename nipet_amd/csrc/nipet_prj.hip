@@ -147,8 +147,8 @@ __device__ inline double rdlane(double v, int l) {
 //    16-byte LDS read. The sums telescope over planes the LOR never enters, so
 //    they are kept in float64, which costs no more instructions than float32 on
 //    this chip (full-rate FP64); a LOR that misses the object is left with
-//    rounding of 1e-16 of the bin's largest line integral and is set to 0
-//    (FZ_SNAP).
+//    rounding of 1e-16 of the bin's largest line integral (of magnitudes) and is
+//    set to 0 (FZ_SNAP).
 //  - Two waves stage the rows of a chunk of FZ_CH segments while the others
 //    cross the chunk before: one barrier a chunk, and no wave does both. The
 //    staging waves wait for memory, so a whole chunk of columns is on its way
@@ -164,9 +164,15 @@ __device__ inline double rdlane(double v, int l) {
 //    only rings r0 < 32 start a LOR. Where a crossing lies (segment, fraction)
 //    is geometry: the table Geom::ev, read through the scalar cache (the vector
 //    unit has enough to do).
+//  - A LOR below FZ_FAINT of that largest one may be small values beside the
+//    rounding of large ones, in a bin that has voxels as small (FZ_SMALL; never
+//    mind attenuation factors, which are exp of it, below FZ_MU, and ratios whose
+//    additive term is larger or whose LOR is below the guard). The LORs of such a
+//    wave and ring difference are walked segment by segment, with the plane
+//    changes from the table.
 //  - Non-finite voxels: a prefix sum would carry them into LORs that do not
-//    touch them. A bin whose totals are not finite is walked segment by
-//    segment instead.
+//    touch them. A bin whose line integrals are not finite in float32 is walked
+//    segment by segment too.
 // Span-1 -> span-N: each output bin sums its LORs in a fixed order from LDS
 // (no atomics, bit-reproducible).
 constexpr int FZ_THREADS = 1024;
@@ -179,7 +185,8 @@ constexpr int FZ_RING = 64;                // rows in LDS, by segment modulo FZ_
 // the ring, its first row again (the row behind the last), and what lanes past
 // ring 63 read (the last of it: where a lane without a plane writes)
 constexpr int FZ_NE = (FZ_RING + 1) * 128 + 64;
-constexpr double FZ_SNAP = 0x1p-44;
+constexpr double FZ_SNAP = 0x1p-44, FZ_FAINT = 0x1p-24;
+constexpr float FZ_SMALL = 0x1p-20f, FZ_MU = 0x1p16f;
 static_assert(2 * FZ_CH + 1 <= FZ_RING, "a chunk is staged while the one before is read");
 static_assert(3 * FZ_CH <= SEG_PAD, "records behind the list are read");
 static_assert(FZ_NE * sizeof(double) >= (2 * LI_MAX + 1) * sizeof(float),
@@ -201,7 +208,9 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
   __shared__ __align__(16) double E[NB][FZ_NE];
   __shared__ double tot[NB][128];
   __shared__ double cend[NB][128];
-  __shared__ float cmax[NB][2];
+  // largest line integral of magnitudes; smallest voxel other than 0, minus 1 (bits
+  // without the sign)
+  __shared__ unsigned cmax[NB][2], cmin[NB][2];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row = blockIdx.x;
@@ -229,9 +238,9 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
 
   // the crossing waves' ring differences, from dmax down in turns: slots 0 .. 2
   // from 32 up (only rings r0 < 32 start a LOR), 3 .. 5 below; -1: none
-  const int cw = wv - FZ_SW, top = min(dmax, 31);
+  const int cw = wv - FZ_SW, top31 = min(dmax, 31);
   int ds[FZ_NS] = {dmax - cw, dmax - 2 * FZ_CW + 1 + cw, dmax - 2 * FZ_CW - cw,
-                   top - cw,  top - 2 * FZ_CW + 1 + cw,  top - 2 * FZ_CW - cw};
+                   top31 - cw, top31 - 2 * FZ_CW + 1 + cw, top31 - 2 * FZ_CW - cw};
 #pragma unroll
   for (int i = 0; i < FZ_NS; i++)
     if (cw < 0 || ds[i] < (i < 3 ? 32 : 0)) ds[i] = -1;
@@ -276,11 +285,13 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
     col1 = t.y;
   };
   double carry[NB];
-  float cmx[NB];
+  float line[NB];    // line integral of the plane's magnitudes so far
+  unsigned xmin[NB];
 #pragma unroll
   for (int b = 0; b < NB; b++) {
     carry[b] = 0.0;
-    cmx[b] = 0.f;
+    line[b] = 0.f;
+    xmin[b] = ~0u;
   }
   // rows first + c + 1 .. first + c + FZ_CH, each read again FZ_PF segments on
   auto stage = [&](int c) {
@@ -293,6 +304,12 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
         const float x1 = __int_as_float(__builtin_amdgcn_update_dpp(
             0, __float_as_int(x0[r][b]), 0x130 /* wave_shl:1 */, 0xf, 0xf, true));
         carry[b] = fma((double)L, (double)x0[r][b] - (double)x1, carry[b]);
+        line[b] = fmaf(L, fabsf(x0[r][b]), line[b]);
+        asm volatile("" : "+v"(line[b]));  // (now, not when the later rows are here too)
+        if constexpr (MODE != 1) {
+          xmin[b] = min(xmin[b], (__float_as_uint(x0[r][b]) << 1) - 1u);
+          asm volatile("" : "+v"(xmin[b]));
+        }
         E[b][slot * 128 + e0] = carry[b];
         if (slot == 0) E[b][FZ_RING * 128 + e0] = carry[b];
       }
@@ -300,8 +317,6 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
     });
     len = len1;
     records(c + 2 * FZ_CH);
-#pragma unroll
-    for (int b = 0; b < NB; b++) cmx[b] = fmaxf(cmx[b], fabsf((float)carry[b]));
   };
   int wn[FZ_NS] = {0, 0, 0, 0, 0, 0};  // slot i: the next crossing's plane offset
   // the next eight crossings of slot i (a list ends in eight past any segment)
@@ -377,6 +392,11 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
       wn[i] = w;
     });
   };
+  // plane offset of ring difference d at the start, rounded down on a tie
+  auto start = [&](int d) {
+    const double t0 = seg[0].s * (2.0 / gp->atn[aw]);
+    return max(__builtin_amdgcn_readfirstlane((int)floor(fma((double)d, t0, 0.5 - 1e-9))), 0);
+  };
   // a chunk is staged while the one before it is crossed: as many barriers on
   // both sides (apart, so that neither side's registers burden the other)
   if (wv < FZ_SW) {
@@ -393,14 +413,12 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
     }
   } else {
     if (nseg > 0) {
-      const double t0 = seg[0].s * (2.0 / gp->atn[aw]);
-      // plane offset at the start, rounded down on a tie, then past the crossings
-      // of earlier segments
+      // plane offset at the start, then past the crossings of earlier segments
       unsigned first_ev[FZ_NS];
 #pragma unroll
       for (int i = 0; i < FZ_NS; i++) {
         const int d = max(ds[i], 0);
-        wn[i] = max(__builtin_amdgcn_readfirstlane((int)floor(fma((double)d, t0, 0.5 - 1e-9))), 0);
+        wn[i] = start(d);
         first_ev[i] = d > 0 ? ev[ev_off(d) + wn[i]].x : ~0u;
       }
 #pragma unroll
@@ -417,21 +435,24 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
   __syncthreads();  // the last chunk's crossings done (the rows' space is used again)
   asm volatile("" ::"v"(touch));
 
-  // C_p(t_end) = sum of the total differences from plane p up, and the largest
-  // magnitude of the prefix sums
-  bool bad = false;
+  // C_p(t_end) = sum of the total differences from plane p up
   if (wv < FZ_SW) {
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-      bad |= own && !isfinite(carry[b]);
-      float m = own ? cmx[b] : 0.f;
-      for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-      if (lane == 0) cmax[b][wv] = m;
+      unsigned m = own ? __float_as_uint(line[b]) : 0u, n = own ? xmin[b] : ~0u;
+      for (int o = 32; o > 0; o >>= 1) {
+        m = max(m, (unsigned)__shfl_xor((int)m, o));
+        n = min(n, (unsigned)__shfl_xor((int)n, o));
+      }
+      if (lane == 0) {
+        cmax[b][wv] = m;
+        cmin[b][wv] = n;
+      }
       if (own) tot[b][pl] = carry[b];
       if (wv == 0 && lane == 63) tot[b][127] = 0.0;
     }
   }
-  const bool slow = __syncthreads_or(bad);
+  __syncthreads();
   if (wv < FZ_SW) {  // wave 0: planes 0 .. 63; wave 1: 64 .. 127; each a suffix sum
 #pragma unroll
     for (int b = 0; b < NB; b++) {
@@ -455,8 +476,26 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
   float *lorv = (float *)&E[0][0];
   static_for<NB>([&](auto bc) {
     constexpr int b = decltype(bc)::value;
-    const double snap = FZ_SNAP * (double)fmaxf(cmax[b][0], cmax[b][1]);
     const double atn = gp->atn[aw];
+    const unsigned um = __builtin_amdgcn_readfirstlane(max(cmax[b][0], cmax[b][1])),
+                   un = __builtin_amdgcn_readfirstlane(min(cmin[b][0], cmin[b][1]));
+    const float top = __uint_as_float(um), small = __uint_as_float((un + 1u) >> 1);
+    const bool slow = !(top < INFINITY);
+    // values up to this are walked; in a ratio without a larger additive term, and
+    // unless all up to it are below the guard (1e-6, at most six LORs a sinogram)
+    const double faint = slow ? INFINITY
+                         : MODE == 1 ? (top > FZ_MU ? FZ_FAINT * top : -1.0)
+                         : small < FZ_SMALL * top && (MODE == 0 || top > 2.f) ? FZ_FAINT * top
+                                                                               : -1.0;
+    const double snap = FZ_SNAP * top;
+    const float *rh = rho + (size_t)aw * gp->nsn * (rho_nb ? nbt : 1) + (rho_nb ? b0 + b : 0);
+    const int rs = rho_nb ? nbt : 1;
+    auto put = [&](int li, double v, float sf) {
+      float f = (float)v * sf;
+      if (MODE == 1) f = expf(-f) * gp->li_nosi[li];
+      lorv[2 * li + (mir ? 1 : 0)] = f;
+    };
+    unsigned redo = 0;  // bit 2 i + k: LORs k of slot i are walked
     if (b > 0) __syncthreads();  // the previous replicate's sums are done
     static_for<FZ_NS>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
@@ -467,46 +506,67 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
       for (int k = 0; k < (i < 3 ? 1 : 2); k++) {
         const int r0 = (lane & 31) + 32 * k;
         const int li = r0 + d <= 63 ? gp->dr_li[d * 64 + r0] : -1;
-        if (li < 0 || (mir && d == 0)) continue;
-        double v;
-        if (slow) {  // segment by segment, only the pieces inside it
-          v = 0.0;
-          double pos = seg[0].s;
-          int w = max((int)floor(fma((double)d, pos * (2.0 / atn), 0.5 - 1e-9)), 0);
-          for (int j = 0; j < nseg; j++) {
-            const double end = j + 1 < nseg ? seg[j + 1].s : seg[j].s + (double)seg[j].len;
-            for (bool in = true; in;) {
-              const double tb = d > 0 ? (w + 0.5) * atn / (2.0 * d) : end;
-              in = tb < end;
-              const double q = in ? tb : end;
-              const int pz = min(max((mir ? 2 * d - w : w) + 2 * r0, 0), NZ - 1);
-              if (q > pos) {
-                v += (q - pos) * (double)img[((int64_t)seg[j].colz + pz) * nbt + b0 + b];
-                pos = q;
-              }
-              w += in ? 1 : 0;
-            }
-          }
-        } else {
-          const int pz = (mir ? 2 * d - wn[i] : wn[i]) + 2 * r0;
-          const double x = acc[i][k][b];
-          v = cend[b][(pz & 1) * 64 + (pz >> 1)] + (mir ? -x : x);
-          if (fabs(v) <= snap) v = 0.0;
+        const bool live = li >= 0 && !(mir && d == 0);
+        const int pz = (mir ? 2 * d - wn[i] : wn[i]) + 2 * r0;
+        const double x = acc[i][k][b];
+        double v = live ? cend[b][(pz & 1) * 64 + (pz >> 1)] + (mir ? -x : x) : 0.0;
+        bool need = live && !(fabs(v) > faint);
+        if (fabs(v) <= snap) v = 0.0;
+        if (MODE == 2 && need && !slow) {
+          const short2 sn = gp->li_sn[li];
+          need = !(fabsf(rh[(size_t)(mir ? sn.y : sn.x) * rs]) > 2.0 * faint);
         }
-        float f = (float)v * sf;
-        if (MODE == 1) f = expf(-f) * gp->li_nosi[li];
-        lorv[2 * li + (mir ? 1 : 0)] = f;
+        if (__builtin_amdgcn_ballot_w64(need)) redo |= 1u << (2 * i + k);
+        if (live) put(li, v, sf);
       }
     });
+    redo = __builtin_amdgcn_readfirstlane(redo);
+    for (; redo; redo &= redo - 1) {
+      const int q = __builtin_ctz(redo), i = (q >> 1) % 3, t = q >= 6 ? top31 : dmax;
+      const int d = i == 0 ? t - cw : i == 1 ? t - 2 * FZ_CW + 1 + cw : t - 2 * FZ_CW - cw;
+      const int r0 = (lane & 31) + 32 * (q & 1);
+      const int li = r0 + d <= 63 ? gp->dr_li[d * 64 + r0] : -1;
+      if (li < 0 || (mir && d == 0)) continue;
+      int w = start(d), j = 0;
+      const uint2s NIPET_CONST *e = ev + ev_off(max(d, 1)) + w;
+      unsigned at = d > 0 ? e->x : ~0u;
+      while ((int)((at & EV_PLACE) >> 10) < first) {
+        at = (++e)->x;
+        w++;
+      }
+      unsigned o = ((mir ? 2 * d - w : w) + 2 * r0) * vb + 4 * b;
+      auto voxel = [&](int j) { return *(const float *)(im + ((unsigned)seg[j].colz * vb + o)); };
+      double v = 0.0, f0 = 0.0;  // f0: the part of segment j that is done
+      while (j < nseg) {
+        // to the next crossing, or to the end
+        const int je = min((int)((at & EV_PLACE) >> 10) - first, nseg);
+        if (j < je) {
+          if (f0 < 1.0 && seg[j].len > 0.f)
+            v += (1.0 - f0) * seg[j].len * (double)voxel(j);
+          f0 = 0.0;
+#pragma unroll 4
+          for (j++; j < je; j++) {
+            const float x = voxel(j);
+            v += seg[j].len > 0.f ? (double)seg[j].len * (double)x : 0.0;
+          }
+        }
+        if (j >= nseg) break;
+        const double f = __hiloint2double(e->y, at & ~EV_PLACE);
+        if (f > f0 && seg[j].len > 0.f)
+          v += (f - f0) * seg[j].len * (double)voxel(j);
+        f0 = fmax(f, f0);
+        o += mir ? 0u - vb : vb;
+        at = (++e)->x;
+      }
+      put(li, v, lor_sfac(2.f * d, gp->vox_z, atn));
+    }
     // the sinogram's members and, in an OSEM update, its counts and additive
     // term: read before the values are complete
     const int nsn = gp->nsn;
     float *out = sino + (size_t)row * nsn * nbt + b0;
     const uint4 *mem = (const uint4 *)gp->sn_mem;
     const int nm = gp->sn_w / 8;  // 16-byte pieces of 8 members per sinogram
-    const float *rh = rho + (size_t)aw * nsn * (rho_nb ? nbt : 1) + (rho_nb ? b0 + b : 0);
     const uint16_t *pr = prompts + (size_t)aw * nsn * nbt + b0 + b;
-    const int rs = rho_nb ? nbt : 1;
     uint4 m4 = make_uint4(0, 0, 0, 0);
     float r = 0.f, y = 0.f;
     auto load = [&](int s) {

@@ -9,7 +9,7 @@ less than a plane, is left out: there their own rounding rules."""
 import numpy as np
 import pytest
 
-from test_gpu_crossings import back, exact_back, rows_of
+from test_gpu_crossings import back, exact, exact_back, project, rows_of
 
 pytestmark = pytest.mark.gpu
 BAR = 1e-5
@@ -105,3 +105,86 @@ def test_staged_non_finite_pair(torch, lib, params, bad):
     assert bool(hit.any()) and not bool(torch.isfinite(got[..., 0][hit]).any())
     assert own(got[..., 0], ref[0], ~hit) < BAR
     assert own(got[..., 1], ref[1], torch.ones_like(hit)) < BAR
+
+
+# --------------------------------------------------------- forward projection
+def voxels(torch, geom, rows, bright, faint, seed):
+    """Image of values about ``faint`` with a few voxels of ``bright`` on the
+    first bins' rays, and the voxels within a plane of those."""
+    g = torch.Generator(device='cuda').manual_seed(seed)
+    img = faint * (0.5 + torch.rand((320, 320, 127), generator=g, device='cuda'))
+    off, col, _, _ = geom.tx_lists()
+    big = torch.zeros(img.shape, dtype=torch.bool, device='cuda')
+    for k, aw in enumerate(rows[:8].tolist()):
+        c = int(col[(off[aw] + off[aw + 1]) // 2])
+        big[c // 320, c % 320, 30 + 8 * k] = True
+    return torch.where(big, torch.full_like(img, bright), img), near(torch, big)
+
+
+@pytest.mark.parametrize('bright,faint', [(1e6, 1e-12), (3.4e38, 1.0), (1.0, 1e-6), (1e30, 1e-30)])
+def test_forward_projection_small_beside_large(torch, lib, params, bright, faint):
+    """LORs that do not touch the large voxels, against the FP64 oracle; in a
+    batch as alone, bit for bit."""
+    from nipet_amd.geom import get_geom
+    geom, rows = get_geom(params), rows_of(torch, 24, 54)
+    img, big = voxels(torch, geom, rows, bright, faint, 3)
+    hit = exact(torch, params, big.float(), rows) > 0
+    got, ref = project(torch, lib, 'nipet_fprj', geom, img, rows), exact(torch, params, img, rows)
+    assert bool(hit.any()) and bool((ref[~hit] > 0).any())
+    assert own(got, ref, ~hit) < BAR
+    assert bool((got[hit] > 0).all())
+    two = torch.stack([torch.rand_like(img), img], 3).contiguous()
+    assert torch.equal(project(torch, lib, 'nipet_fprj_b', geom, two, rows, nb=2)[..., 1], got)
+
+
+@pytest.mark.parametrize('bright', [1e7, 3.4e38])
+def test_attenuation_beside_large(torch, lib, params, bright):
+    """Attenuation factors of LORs that do not touch the large voxels."""
+    from nipet_amd.geom import get_geom
+    geom, rows = get_geom(params), rows_of(torch, 24, 55)
+    mu, big = voxels(torch, geom, rows, bright, 0.01, 4)
+    hit = exact(torch, params, big.float(), rows) > 0
+    got = project(torch, lib, 'nipet_fprj', geom, mu, rows, 1)
+    assert own(got, exact(torch, params, mu, rows, 1), ~hit) < BAR
+    assert bool((got[hit] < 1).all())
+
+
+@pytest.mark.parametrize('bright,faint,add', [(1e6, 1e-5, 0.0), (3.4e38, 1e-2, 0.0),
+                                              (1e6, 1e-5, 1e-3), (1e6, 1e-5, 1e2)])
+def test_ratio_beside_large(torch, lib, params, bright, faint, add):
+    """The OSEM ratio of LORs that do not touch the large voxels, without and with
+    an additive term."""
+    from nipet_amd.geom import get_geom
+    geom, rows = get_geom(params), rows_of(torch, 24, 56)
+    img, big = voxels(torch, geom, rows, bright, faint, 5)
+    hit = exact(torch, params, big.float(), rows) > 0
+    prompts = torch.full((geom.naw, geom.nsn), 3, dtype=torch.int32, device='cuda').to(torch.uint16)
+    rho = torch.full((geom.naw, geom.nsn), add, device='cuda')
+    mask = torch.ones((320, 320, 127), dtype=torch.uint8, device='cuda')
+    sens, wimg = torch.ones((320, 320, 127), device='cuda'), torch.empty_like(img)
+    got, upd = torch.zeros((len(rows), geom.nsn), device='cuda'), img.clone()
+    lib.check(lib.lib().nipet_osem_subset(
+        geom.handle, lib.ptr(upd), lib.ptr(prompts), lib.ptr(rho), lib.ptr(sens),
+        lib.ptr(mask), None, lib.ptr(rows), len(rows), lib.ptr(got), lib.ptr(wimg),
+        lib.stream_handle()), 'nipet_osem_subset')
+    ref = exact(torch, params, img, rows).double() + add
+    assert float(ref[~hit].min()) > 1e-5  # (far from the guard)
+    assert own(got, 3.0 / ref, ~hit) < BAR
+
+
+@pytest.mark.parametrize('bad', [float('inf'), float('nan')])
+def test_forward_non_finite_pair(torch, lib, params, bad):
+    """Two images: a non-finite voxel changes nothing in the other image, and in
+    its own the LORs that touch it."""
+    from nipet_amd.geom import get_geom
+    geom, rows = get_geom(params), rows_of(torch, 24, 57)
+    img, big = voxels(torch, geom, rows, bad, 1.0, 6)
+    hit = exact(torch, params, big.float(), rows) > 0
+    clean = torch.where(torch.isfinite(img), img, torch.zeros_like(img))
+    two = torch.stack([img, torch.rand_like(img)], 3).contiguous()
+    got = project(torch, lib, 'nipet_fprj_b', geom, two, rows, nb=2)
+    assert torch.equal(got[..., 1], project(torch, lib, 'nipet_fprj', geom,
+                                            two[..., 1].contiguous(), rows))
+    assert own(got[..., 0], exact(torch, params, clean, rows), ~hit) < BAR
+    touch = exact(torch, params, (~torch.isfinite(img)).float(), rows) > 0
+    assert not bool(torch.isfinite(got[..., 0][touch]).any())
