@@ -4,6 +4,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <memory>
+#include <vector>
+
 #include "nipet_hip.h"
 
 namespace nipet {
@@ -52,13 +55,20 @@ struct GeomView {
   float vox_z;
 };
 
-// Geometry resident on one device. Transaxial intersection lists in CSR form:
-// segments of ray aw are seg[off[aw] .. off[aw+1]).
-struct Geom {
-  int device = 0;
-  int naw = 0, nli = 0, nsn = 0, ncrs = 0, ndirect = 0;
+// The rays of a scanner on one device: transaxial intersection lists in CSR form
+// (segments of ray aw are seg[off[aw] .. off[aw+1])) and the z crossings along
+// them, 4.3 GB for 68,516 bins of 272 segments. They depend on the crystals, the
+// grid and the largest ring difference, not on spans or sinograms: geometries of
+// the same rays share them (rays_get).
+struct Rays {
+  // what they are made of
+  int device = 0, naw = 0, dmax = 0;  // dmax: largest ring difference d
+  float vox_xy = 0.f, tfov2 = 0.f;
+  std::vector<float> crs;
+  std::vector<int16_t> s2c;
+
   int64_t nseg = 0;
-  float vox_z = 0.203125f;
+  int maxseg = 0;            // longest list
   int32_t *off = nullptr;    // [naw+1]
   SegRec *seg = nullptr;     // [nseg]
   double *atn = nullptr;     // [naw] crystal-to-crystal transaxial distance
@@ -69,6 +79,25 @@ struct Geom {
   // with its low 20 bits (2^-32 of it) replaced by segment << 10 | ev_phi(w);
   // segment 1023 past the end of the list
   uint2 *ev = nullptr;
+  // z crossings in the order of the back projector's walk (nseg_ev entries, see
+  // bp_event) and the first entry of every segment [nseg + 1]
+  uint2 *bp_ev = nullptr;
+  uint32_t *bp_off = nullptr;
+  // segments by voxel column (CSR): bin << 10 | segment of the bin's list, ascending
+  int32_t *col_off = nullptr;   // [NX * NY + 1]
+  uint32_t *col_ent = nullptr;  // [nseg]
+
+  Rays() = default;
+  Rays(const Rays &) = delete;
+  ~Rays();
+};
+
+// Geometry resident on one device: rays, and the sinograms their LORs belong to.
+struct Geom {
+  int device = 0;
+  int naw = 0, nli = 0, nsn = 0, ncrs = 0, ndirect = 0;
+  std::shared_ptr<const Rays> rays;
+  float vox_z = 0.203125f;
   float2 *li_z = nullptr;    // [nli] (zeta_a at t=0, zeta_b - zeta_a) in z-voxel units
   short2 *li_sn = nullptr;   // [nli] output sinogram of LOR a and of its mirror b
   float *li_nosi = nullptr;  // [nli] 1 / (span-1 LORs per output sinogram)
@@ -87,14 +116,6 @@ struct Geom {
   // back-projector LOR table [BP_TN]: at 65 d + r0 the sinograms of LOR (r0, d)
   // and (<< 16) of its mirror; nsn where there is none
   uint32_t *bp_tab = nullptr;
-  // z crossings in the order of the back projector's walk (nseg_ev entries, see
-  // bp_event) and the first entry of every segment [nseg + 1]
-  uint2 *bp_ev = nullptr;
-  uint32_t *bp_off = nullptr;
-  // segments by voxel column (CSR): bin << 10 | segment of the bin's list, ascending
-  int32_t *col_off = nullptr;   // [NX * NY + 1]
-  uint32_t *col_ent = nullptr;  // [nseg]
-  int maxseg = 0;               // longest list
   GeomView view = {};           // the pointers above, and
   GeomView *dview = nullptr;    // its copy on the device
 };
@@ -108,7 +129,7 @@ constexpr int BP_TN = 65 * (BP_MAXD + 1) + 64;
 // Plane offset of the LORs of one ring difference at t = s (m = 2 d / atn).
 __device__ inline int plane_offset(double m, double s) { return (int)floor(fma(m, s, 0.5)); }
 
-// Entry of Geom::bp_ev: the LORs of ring difference d pass from plane offset w
+// Entry of Rays::bp_ev: the LORs of ring difference d pass from plane offset w
 // to w + 1, beta before the segment's end. A float64 +beta (w even) or -beta
 // (odd) with its low 23 bits (2^-30 of beta) replaced by: 1 for the segment's
 // last entry, 4 D, and d << 16. The LORs are at entries D + i, D + i + 1 (one
@@ -128,9 +149,9 @@ __device__ inline uint2 bp_event(int d, int w, double beta, bool last) {
 // Position of plane w in the forward projector's LDS rows (64 even planes, then
 // 64 odd ones, of 8 bytes), in bytes.
 __host__ __device__ constexpr int ev_phi(int w) { return ((w & 1) << 9) + ((w >> 1) << 3); }
-constexpr uint32_t EV_PLACE = 0xfffffu;  // the place in an entry of Geom::ev
+constexpr uint32_t EV_PLACE = 0xfffffu;  // the place in an entry of Rays::ev
 static_assert(MAX_SEG < 1023, "segments in 10 bits");
-// Crossings of ring difference d in Geom::ev: 2 d, and eight that lie past any
+// Crossings of ring difference d in Rays::ev: 2 d, and eight that lie past any
 // segment (eight are read at a time).
 __host__ __device__ constexpr int ev_off(int d) { return (d - 1) * (d + 8); }
 

@@ -21,6 +21,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <memory>
 #include <mutex>
 #include <vector>
 
@@ -235,7 +236,7 @@ __global__ void k_tx_lists(const float *crs, const short2 *s2c, int naw, double 
   }
 }
 
-// z crossings of every ray (Geom::ev), one workgroup per bin: a binary search
+// z crossings of every ray (Rays::ev), one workgroup per bin: a binary search
 // of t in the bin's segment starts per crossing. (Crossings before the list
 // get its start; no walk reads them.)
 __global__ __launch_bounds__(256) void k_events(const int32_t *__restrict__ off,
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(256) void k_events(const int32_t *__restrict__ off,
   }
 }
 
-// Geom::bp_ev of one bin per wave, lane d its ring difference d: the number of
+// Rays::bp_ev of one bin per wave, lane d its ring difference d: the number of
 // entries (ev NULL), or the entries from base[bin] on and the segments' offsets.
 __global__ __launch_bounds__(64) void k_bp_events(const int32_t *__restrict__ off,
                                                   const SegRec *__restrict__ seg,
@@ -308,7 +309,7 @@ __global__ __launch_bounds__(64) void k_bp_events(const int32_t *__restrict__ of
   if (!ev && lane == 0) base[aw] = pos;
 }
 
-// Segments by voxel column (Geom::col_off, col_ent): counts per column, then
+// Segments by voxel column (Rays::col_off, col_ent): counts per column, then
 // entries in any order, then each column's entries in ascending order (the rank
 // of every entry among the column's, n^2 comparisons of a few hundred).
 __global__ void k_col_count(const SegRec *__restrict__ seg, int64_t n, int32_t *cnt) {
@@ -408,11 +409,188 @@ int nipet_prof_read(int kernel, double *total_ms, int64_t *count) {
 
 static void geom_free(Geom *g) {
   // teardown: a failing free leaves nothing to undo
-  void *bufs[] = {g->off,   g->seg,    g->atn,    g->lmax,   g->li_z,   g->li_sn,
-                  g->li_nosi, g->dr_li, g->sn_mem, g->fp_slot, g->bp_tab, g->bp_ev,
-                  g->bp_off, g->ev, g->dview,
-                  g->col_off, g->col_ent};
+  void *bufs[] = {g->li_z, g->li_sn, g->li_nosi, g->dr_li, g->sn_mem, g->fp_slot, g->bp_tab,
+                  g->dview};
   for (void *p : bufs) (void)hipFree(p);
+}
+
+nipet::Rays::~Rays() {
+  void *bufs[] = {off, seg, atn, lmax, ev, bp_ev, bp_off, col_off, col_ent};
+  for (void *p : bufs) (void)hipFree(p);
+}
+
+// The lists and crossings of r's rays (r->device, naw and dmax are set).
+static int rays_build(const NipetGeomDesc *d, Rays *r) {
+  float *d_crs = nullptr;
+  short2 *d_s2c = nullptr;
+  int32_t *d_cnt = nullptr;
+  int *d_err = nullptr;
+  // the build's temporaries are freed on every return path
+  struct Tmp {
+    void **p[4];
+    ~Tmp() {
+      for (void **q : p) (void)hipFree(*q);
+    }
+  } tmp{{(void **)&d_crs, (void **)&d_s2c, (void **)&d_cnt, (void **)&d_err}};
+  NIPET_HIP(hipMalloc(&d_crs, d->ncrs * 4 * sizeof(float)));
+  NIPET_HIP(hipMalloc(&d_s2c, d->naw * sizeof(short2)));
+  NIPET_HIP(hipMalloc(&d_cnt, d->naw * sizeof(int32_t)));
+  NIPET_HIP(hipMalloc(&d_err, sizeof(int)));
+  NIPET_HIP(hipMalloc(&r->atn, d->naw * sizeof(double)));
+  NIPET_HIP(hipMalloc(&r->lmax, d->naw * sizeof(float)));
+  NIPET_HIP(hipMalloc(&r->off, (d->naw + 1) * sizeof(int32_t)));
+  NIPET_HIP(hipMemcpy(d_crs, d->crs, d->ncrs * 4 * sizeof(float), hipMemcpyHostToDevice));
+  NIPET_HIP(hipMemcpy(d_s2c, d->s2c, d->naw * sizeof(short2), hipMemcpyHostToDevice));
+  NIPET_HIP(hipMemset(d_err, 0, sizeof(int)));
+  NIPET_HIP(hipMemset(r->lmax, 0, d->naw * sizeof(float)));
+  int nb = (d->naw + 255) / 256;
+  k_tx_lists<<<nb, 256>>>(d_crs, d_s2c, d->naw, (double)d->vox_xy, (double)d->tfov2, NZ,
+                          nullptr, d_cnt, nullptr, r->atn, r->lmax, d_err);
+  NIPET_HIP(hipGetLastError());
+  std::vector<int32_t> cnt(d->naw);
+  int herr = 0;
+  NIPET_HIP(hipMemcpy(cnt.data(), d_cnt, d->naw * sizeof(int32_t), hipMemcpyDeviceToHost));
+  NIPET_HIP(hipMemcpy(&herr, d_err, sizeof(int), hipMemcpyDeviceToHost));
+  if (herr) {
+    set_error("transaxial ray left the image grid (inconsistent geometry)");
+    return NIPET_EINVAL;
+  }
+  std::vector<int32_t> off(d->naw + 1);
+  int64_t tot = 0;
+  for (int i = 0; i < d->naw; i++) {
+    if (cnt[i] > MAX_SEG) {  // the projectors stage one ray's list in LDS
+      set_error("transaxial ray %d has %d segments (at most %d)", i, cnt[i], MAX_SEG);
+      return NIPET_EINVAL;
+    }
+    off[i] = (int32_t)tot;
+    tot += cnt[i];
+  }
+  off[d->naw] = (int32_t)tot;
+  if (tot >= INT32_MAX) {
+    set_error("too many transaxial segments");
+    return NIPET_EINVAL;
+  }
+  r->nseg = tot;
+  NIPET_HIP(hipMemcpy(r->off, off.data(), (d->naw + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
+  // the projectors read whole chunks of records: padded behind the last list
+  NIPET_HIP(hipMalloc(&r->seg, (tot + SEG_PAD) * sizeof(SegRec)));
+  NIPET_HIP(hipMemset(r->seg + tot, 0, SEG_PAD * sizeof(SegRec)));
+  k_tx_lists<<<nb, 256>>>(d_crs, d_s2c, d->naw, (double)d->vox_xy, (double)d->tfov2, NZ, r->off,
+                          nullptr, r->seg, nullptr, r->lmax, d_err);
+  NIPET_HIP(hipGetLastError());
+  {  // eight crossings are read at a time, also where there are none (dmax 0)
+    const size_t ne = ev_off(r->dmax + 1);
+    NIPET_HIP(hipMalloc(&r->ev, (d->naw * ne + 8) * sizeof(uint2)));
+    NIPET_HIP(hipMemset(r->ev + d->naw * ne, 0xff, 8 * sizeof(uint2)));
+    if (ne > 0) k_events<<<d->naw, 256>>>(r->off, r->seg, r->atn, r->dmax, r->ev);
+    NIPET_HIP(hipGetLastError());
+  }
+  NIPET_HIP(hipDeviceSynchronize());
+  // the projectors split a segment into at most three z pieces: no segment may
+  // span two z-boundary spacings atn / (2 dmax) of the steepest LOR
+  {
+    std::vector<float> lm(d->naw);
+    std::vector<double> at(d->naw);
+    NIPET_HIP(hipMemcpy(lm.data(), r->lmax, d->naw * sizeof(float), hipMemcpyDeviceToHost));
+    NIPET_HIP(hipMemcpy(at.data(), r->atn, d->naw * sizeof(double), hipMemcpyDeviceToHost));
+    for (int i = 0; i < d->naw; i++)
+      if ((double)lm[i] * 2.0 * r->dmax >= 1.99 * at[i]) {
+        set_error("transaxial bin %d: segments cross more than two z-planes", i);
+        return NIPET_EINVAL;
+      }
+  }
+  {
+    uint32_t *base = nullptr;
+    struct Tmp3 {
+      uint32_t **p;
+      ~Tmp3() { (void)hipFree(*p); }
+    } tmp3{&base};
+    NIPET_HIP(hipMalloc(&base, d->naw * sizeof(uint32_t)));
+    k_bp_events<<<d->naw, 64>>>(r->off, r->seg, r->atn, r->dmax, base, nullptr, nullptr);
+    NIPET_HIP(hipGetLastError());
+    std::vector<uint32_t> be(d->naw);
+    NIPET_HIP(hipMemcpy(be.data(), base, d->naw * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    uint64_t ne = 0;
+    for (uint32_t &b : be) {
+      const uint32_t c = b;
+      b = (uint32_t)ne;
+      ne += c;
+    }
+    if (ne > UINT32_MAX) {
+      set_error("too many z crossings");
+      return NIPET_EINVAL;
+    }
+    const uint32_t end = (uint32_t)ne;
+    // (entries are read in eights, one eight ahead)
+    NIPET_HIP(hipMalloc(&r->bp_ev, (ne + 24) * sizeof(uint2)));
+    NIPET_HIP(hipMemset(r->bp_ev + ne, 0, 24 * sizeof(uint2)));
+    NIPET_HIP(hipMalloc(&r->bp_off, (tot + 1) * sizeof(uint32_t)));
+    NIPET_HIP(hipMemcpy(r->bp_off + tot, &end, sizeof(end), hipMemcpyHostToDevice));
+    NIPET_HIP(hipMemcpy(base, be.data(), d->naw * sizeof(uint32_t), hipMemcpyHostToDevice));
+    k_bp_events<<<d->naw, 64>>>(r->off, r->seg, r->atn, r->dmax, base, r->bp_ev, r->bp_off);
+    NIPET_HIP(hipGetLastError());
+    NIPET_HIP(hipDeviceSynchronize());
+  }
+  {
+    for (int i = 0; i < d->naw; i++) r->maxseg = std::max(r->maxseg, (int)cnt[i]);
+    int32_t *cur = nullptr;
+    uint32_t *ent = nullptr;
+    struct Tmp2 {
+      void **p[2];
+      ~Tmp2() {
+        for (void **q : p) (void)hipFree(*q);
+      }
+    } tmp2{{(void **)&cur, (void **)&ent}};
+    const size_t nc = NX * NY;
+    NIPET_HIP(hipMalloc(&cur, nc * sizeof(int32_t)));
+    NIPET_HIP(hipMalloc(&ent, (tot + 1) * sizeof(uint32_t)));
+    NIPET_HIP(hipMalloc(&r->col_off, (nc + 1) * sizeof(int32_t)));
+    NIPET_HIP(hipMalloc(&r->col_ent, (tot + 1) * sizeof(uint32_t)));
+    NIPET_HIP(hipMemset(cur, 0, nc * sizeof(int32_t)));
+    if (tot > 0) k_col_count<<<(unsigned)((tot + 255) / 256), 256>>>(r->seg, tot, cur);
+    std::vector<int32_t> co(nc + 1, 0);
+    NIPET_HIP(hipMemcpy(co.data() + 1, cur, nc * sizeof(int32_t), hipMemcpyDeviceToHost));
+    for (size_t i = 0; i < nc; i++) co[i + 1] += co[i];
+    NIPET_HIP(hipMemcpy(r->col_off, co.data(), (nc + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
+    NIPET_HIP(hipMemcpy(cur, co.data(), nc * sizeof(int32_t), hipMemcpyHostToDevice));
+    k_col_fill<<<d->naw, 256>>>(r->off, r->seg, d->naw, cur, ent);
+    k_col_sort<<<(unsigned)nc, 64>>>(r->col_off, ent, r->col_ent);
+    NIPET_HIP(hipGetLastError());
+    NIPET_HIP(hipDeviceSynchronize());
+  }
+  return NIPET_OK;
+}
+
+// The rays of d up to ring difference dmax: those of a living geometry, or new
+// ones. (The list holds no rays of its own; one build at a time.)
+static int rays_get(const NipetGeomDesc *d, int device, int dmax,
+                    std::shared_ptr<const Rays> &out) {
+  static std::mutex mu;
+  static std::vector<std::weak_ptr<const Rays>> known;
+  auto r = std::make_shared<Rays>();
+  r->device = device;
+  r->naw = d->naw;
+  r->dmax = dmax;
+  r->vox_xy = d->vox_xy;
+  r->tfov2 = d->tfov2;
+  r->crs.assign(d->crs, d->crs + 4 * (size_t)d->ncrs);
+  r->s2c.assign(d->s2c, d->s2c + 2 * (size_t)d->naw);
+  std::lock_guard<std::mutex> lk(mu);
+  known.erase(std::remove_if(known.begin(), known.end(), [](auto &w) { return w.expired(); }),
+              known.end());
+  for (auto &w : known) {
+    auto k = w.lock();
+    if (k && k->device == r->device && k->dmax == r->dmax && k->vox_xy == r->vox_xy &&
+        k->tfov2 == r->tfov2 && k->s2c == r->s2c && k->crs == r->crs) {
+      out = k;
+      return NIPET_OK;
+    }
+  }
+  const int rc = rays_build(d, r.get());
+  if (rc) return rc;
+  known.push_back(r);
+  out = r;
+  return NIPET_OK;
 }
 
 static int geom_build(const NipetGeomDesc *d, NipetGeom *g) {
@@ -543,161 +721,26 @@ static int geom_build(const NipetGeomDesc *d, NipetGeom *g) {
   NIPET_HIP(hipMemcpy(g->li_sn, lisn.data(), d->nli * sizeof(short2), hipMemcpyHostToDevice));
   NIPET_HIP(hipMemcpy(g->li_nosi, linos.data(), d->nli * sizeof(float), hipMemcpyHostToDevice));
 
-  // transaxial lists
-  float *d_crs = nullptr;
-  short2 *d_s2c = nullptr;
-  int32_t *d_cnt = nullptr;
-  int *d_err = nullptr;
-  // the build's temporaries are freed on every return path
-  struct Tmp {
-    void **p[4];
-    ~Tmp() {
-      for (void **q : p) (void)hipFree(*q);
-    }
-  } tmp{{(void **)&d_crs, (void **)&d_s2c, (void **)&d_cnt, (void **)&d_err}};
-  NIPET_HIP(hipMalloc(&d_crs, d->ncrs * 4 * sizeof(float)));
-  NIPET_HIP(hipMalloc(&d_s2c, d->naw * sizeof(short2)));
-  NIPET_HIP(hipMalloc(&d_cnt, d->naw * sizeof(int32_t)));
-  NIPET_HIP(hipMalloc(&d_err, sizeof(int)));
-  NIPET_HIP(hipMalloc(&g->atn, d->naw * sizeof(double)));
-  NIPET_HIP(hipMalloc(&g->lmax, d->naw * sizeof(float)));
-  NIPET_HIP(hipMalloc(&g->off, (d->naw + 1) * sizeof(int32_t)));
-  NIPET_HIP(hipMemcpy(d_crs, d->crs, d->ncrs * 4 * sizeof(float), hipMemcpyHostToDevice));
-  NIPET_HIP(hipMemcpy(d_s2c, d->s2c, d->naw * sizeof(short2), hipMemcpyHostToDevice));
-  NIPET_HIP(hipMemset(d_err, 0, sizeof(int)));
-  NIPET_HIP(hipMemset(g->lmax, 0, d->naw * sizeof(float)));
-  int nb = (d->naw + 255) / 256;
-  k_tx_lists<<<nb, 256>>>(d_crs, d_s2c, d->naw, (double)d->vox_xy, (double)d->tfov2, NZ,
-                          nullptr, d_cnt, nullptr, g->atn, g->lmax, d_err);
-  NIPET_HIP(hipGetLastError());
-  std::vector<int32_t> cnt(d->naw);
-  int herr = 0;
-  NIPET_HIP(hipMemcpy(cnt.data(), d_cnt, d->naw * sizeof(int32_t), hipMemcpyDeviceToHost));
-  NIPET_HIP(hipMemcpy(&herr, d_err, sizeof(int), hipMemcpyDeviceToHost));
-  if (herr) {
-    set_error("transaxial ray left the image grid (inconsistent geometry)");
-    return NIPET_EINVAL;
-  }
-  std::vector<int32_t> off(d->naw + 1);
-  int64_t tot = 0;
-  for (int i = 0; i < d->naw; i++) {
-    if (cnt[i] > MAX_SEG) {  // the projectors stage one ray's list in LDS
-      set_error("transaxial ray %d has %d segments (at most %d)", i, cnt[i], MAX_SEG);
-      return NIPET_EINVAL;
-    }
-    off[i] = (int32_t)tot;
-    tot += cnt[i];
-  }
-  off[d->naw] = (int32_t)tot;
-  if (tot >= INT32_MAX) {
-    set_error("too many transaxial segments");
-    return NIPET_EINVAL;
-  }
-  g->nseg = tot;
-  NIPET_HIP(hipMemcpy(g->off, off.data(), (d->naw + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
-  // the projectors read whole chunks of records: padded behind the last list
-  NIPET_HIP(hipMalloc(&g->seg, (tot + SEG_PAD) * sizeof(SegRec)));
-  NIPET_HIP(hipMemset(g->seg + tot, 0, SEG_PAD * sizeof(SegRec)));
-  k_tx_lists<<<nb, 256>>>(d_crs, d_s2c, d->naw, (double)d->vox_xy, (double)d->tfov2, NZ, g->off,
-                          nullptr, g->seg, nullptr, g->lmax, d_err);
-  NIPET_HIP(hipGetLastError());
-  {  // eight crossings are read at a time, also where there are none (dmax 0)
-    const size_t ne = ev_off(g->dmax + 1);
-    NIPET_HIP(hipMalloc(&g->ev, (d->naw * ne + 8) * sizeof(uint2)));
-    NIPET_HIP(hipMemset(g->ev + d->naw * ne, 0xff, 8 * sizeof(uint2)));
-    if (ne > 0) k_events<<<d->naw, 256>>>(g->off, g->seg, g->atn, g->dmax, g->ev);
-    NIPET_HIP(hipGetLastError());
-  }
-  NIPET_HIP(hipDeviceSynchronize());
-  // the projectors split a segment into at most three z pieces: no segment may
-  // span two z-boundary spacings atn / (2 dmax) of the steepest LOR
-  {
-    std::vector<float> lm(d->naw);
-    std::vector<double> at(d->naw);
-    NIPET_HIP(hipMemcpy(lm.data(), g->lmax, d->naw * sizeof(float), hipMemcpyDeviceToHost));
-    NIPET_HIP(hipMemcpy(at.data(), g->atn, d->naw * sizeof(double), hipMemcpyDeviceToHost));
-    for (int i = 0; i < d->naw; i++)
-      if ((double)lm[i] * 2.0 * g->dmax >= 1.99 * at[i]) {
-        set_error("transaxial bin %d: segments cross more than two z-planes", i);
-        return NIPET_EINVAL;
-      }
-  }
-  {
-    uint32_t *base = nullptr;
-    struct Tmp3 {
-      uint32_t **p;
-      ~Tmp3() { (void)hipFree(*p); }
-    } tmp3{&base};
-    NIPET_HIP(hipMalloc(&base, d->naw * sizeof(uint32_t)));
-    k_bp_events<<<d->naw, 64>>>(g->off, g->seg, g->atn, g->dmax, base, nullptr, nullptr);
-    NIPET_HIP(hipGetLastError());
-    std::vector<uint32_t> be(d->naw);
-    NIPET_HIP(hipMemcpy(be.data(), base, d->naw * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    uint64_t ne = 0;
-    for (uint32_t &b : be) {
-      const uint32_t c = b;
-      b = (uint32_t)ne;
-      ne += c;
-    }
-    if (ne > UINT32_MAX) {
-      set_error("too many z crossings");
-      return NIPET_EINVAL;
-    }
-    const uint32_t end = (uint32_t)ne;
-    // (entries are read in eights, one eight ahead)
-    NIPET_HIP(hipMalloc(&g->bp_ev, (ne + 24) * sizeof(uint2)));
-    NIPET_HIP(hipMemset(g->bp_ev + ne, 0, 24 * sizeof(uint2)));
-    NIPET_HIP(hipMalloc(&g->bp_off, (tot + 1) * sizeof(uint32_t)));
-    NIPET_HIP(hipMemcpy(g->bp_off + tot, &end, sizeof(end), hipMemcpyHostToDevice));
-    NIPET_HIP(hipMemcpy(base, be.data(), d->naw * sizeof(uint32_t), hipMemcpyHostToDevice));
-    k_bp_events<<<d->naw, 64>>>(g->off, g->seg, g->atn, g->dmax, base, g->bp_ev, g->bp_off);
-    NIPET_HIP(hipGetLastError());
-    NIPET_HIP(hipDeviceSynchronize());
-  }
-  {
-    for (int i = 0; i < d->naw; i++) g->maxseg = std::max(g->maxseg, (int)cnt[i]);
-    int32_t *cur = nullptr;
-    uint32_t *ent = nullptr;
-    struct Tmp2 {
-      void **p[2];
-      ~Tmp2() {
-        for (void **q : p) (void)hipFree(*q);
-      }
-    } tmp2{{(void **)&cur, (void **)&ent}};
-    const size_t nc = NX * NY;
-    NIPET_HIP(hipMalloc(&cur, nc * sizeof(int32_t)));
-    NIPET_HIP(hipMalloc(&ent, (tot + 1) * sizeof(uint32_t)));
-    NIPET_HIP(hipMalloc(&g->col_off, (nc + 1) * sizeof(int32_t)));
-    NIPET_HIP(hipMalloc(&g->col_ent, (tot + 1) * sizeof(uint32_t)));
-    NIPET_HIP(hipMemset(cur, 0, nc * sizeof(int32_t)));
-    if (tot > 0) k_col_count<<<(unsigned)((tot + 255) / 256), 256>>>(g->seg, tot, cur);
-    std::vector<int32_t> co(nc + 1, 0);
-    NIPET_HIP(hipMemcpy(co.data() + 1, cur, nc * sizeof(int32_t), hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < nc; i++) co[i + 1] += co[i];
-    NIPET_HIP(hipMemcpy(g->col_off, co.data(), (nc + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
-    NIPET_HIP(hipMemcpy(cur, co.data(), nc * sizeof(int32_t), hipMemcpyHostToDevice));
-    k_col_fill<<<d->naw, 256>>>(g->off, g->seg, d->naw, cur, ent);
-    k_col_sort<<<(unsigned)nc, 64>>>(g->col_off, ent, g->col_ent);
-    NIPET_HIP(hipGetLastError());
-    NIPET_HIP(hipDeviceSynchronize());
-  }
+  const int rc = rays_get(d, g->device, g->dmax, g->rays);
+  if (rc) return rc;
+  const Rays *r = g->rays.get();
   GeomView &v = g->view;
-  v.off = g->off;
-  v.seg = g->seg;
-  v.atn = g->atn;
-  v.ev = g->ev;
-  v.lmax = g->lmax;
+  v.off = r->off;
+  v.seg = r->seg;
+  v.atn = r->atn;
+  v.ev = r->ev;
+  v.lmax = r->lmax;
   v.li_z = g->li_z;
   v.li_sn = g->li_sn;
   v.li_nosi = g->li_nosi;
   v.dr_li = g->dr_li;
   v.sn_mem = g->sn_mem;
   v.bp_tab = g->bp_tab;
-  v.bp_ev = g->bp_ev;
-  v.bp_off = g->bp_off;
-  v.col_off = g->col_off;
-  v.col_ent = g->col_ent;
-  v.maxseg = g->maxseg;
+  v.bp_ev = r->bp_ev;
+  v.bp_off = r->bp_off;
+  v.col_off = r->col_off;
+  v.col_ent = r->col_ent;
+  v.maxseg = r->maxseg;
   v.fp_slot = g->fp_slot;
   v.fp_nslot = g->fp_nslot;
   v.naw = g->naw;
@@ -750,7 +793,7 @@ int nipet_geom_info(const NipetGeom *g, int *naw, int64_t *nseg_total, int *nli,
     return NIPET_EINVAL;
   }
   if (naw) *naw = g->naw;
-  if (nseg_total) *nseg_total = g->nseg;
+  if (nseg_total) *nseg_total = g->rays->nseg;
   if (nli) *nli = g->nli;
   if (nsn) *nsn = g->nsn;
   return NIPET_OK;
@@ -763,7 +806,7 @@ int nipet_bins_longest_first(const NipetGeom *g, const int32_t *subs, int n, int
     return NIPET_EINVAL;
   }
   if (n == 0) return NIPET_OK;
-  k_bins_longest_first<<<1, 1024, 0, (hipStream_t)stream>>>(g->off, g->naw, subs, n, out);
+  k_bins_longest_first<<<1, 1024, 0, (hipStream_t)stream>>>(g->rays->off, g->naw, subs, n, out);
   NIPET_HIP(hipGetLastError());
   return NIPET_OK;
 }
@@ -775,12 +818,13 @@ int nipet_tx_lists(const NipetGeom *g, int64_t *offsets, int32_t *col, float *t,
     return NIPET_EINVAL;
   }
   std::vector<int32_t> off(g->naw + 1);
-  NIPET_HIP(hipMemcpy(off.data(), g->off, (g->naw + 1) * sizeof(int32_t), hipMemcpyDeviceToHost));
+  NIPET_HIP(hipMemcpy(off.data(), g->rays->off, (g->naw + 1) * sizeof(int32_t), hipMemcpyDeviceToHost));
   for (int i = 0; i <= g->naw; i++) offsets[i] = off[i];
   if (!lists) return NIPET_OK;
-  std::vector<SegRec> sg(g->nseg);
-  NIPET_HIP(hipMemcpy(sg.data(), g->seg, g->nseg * sizeof(SegRec), hipMemcpyDeviceToHost));
-  for (int64_t k = 0; k < g->nseg; k++) {
+  std::vector<SegRec> sg(g->rays->nseg);
+  NIPET_HIP(hipMemcpy(sg.data(), g->rays->seg, g->rays->nseg * sizeof(SegRec),
+                      hipMemcpyDeviceToHost));
+  for (int64_t k = 0; k < g->rays->nseg; k++) {
     col[k] = sg[k].colz / NZ;
     t[k] = (float)sg[k].s;
     len[k] = sg[k].len;

@@ -162,7 +162,7 @@ __device__ inline double rdlane(double v, int l) {
 //  - The crossing waves take the ring differences from the largest down in
 //    turns, so that each has about the same number of crossings. From d = 32 on
 //    only rings r0 < 32 start a LOR. Where a crossing lies (segment, fraction)
-//    is geometry: the table Geom::ev, read through the scalar cache (the vector
+//    is geometry: the table Rays::ev, read through the scalar cache (the vector
 //    unit has enough to do).
 //  - A LOR below FZ_FAINT of that largest one may be small values beside the
 //    rounding of large ones, in a bin that has voxels as small (FZ_SMALL; never
@@ -1638,7 +1638,7 @@ static thread_local struct {
 constexpr int BP_PASS = 8192, BP_STAGE_MIN = 1536;
 
 static int64_t bp_scratch_bytes(const Geom *g, int rows, int nb) {
-  return (int64_t)g->naw * 8 + BP_NAW / 8 + (int64_t)rows * 4 + 256 + (int64_t)rows * g->maxseg * 512 * nb;
+  return (int64_t)g->naw * 8 + BP_NAW / 8 + (int64_t)rows * 4 + 256 + (int64_t)rows * g->rays->maxseg * 512 * nb;
 }
 
 // One sub-batch of width NB into img (overwritten in its replicates' places).

@@ -2,9 +2,10 @@
 
 One ``NipetGeom`` per (scanner parameters, span, device) is built on first use
 and cached: the FP64 transaxial intersection lists of all 68,516 transaxial
-bins are computed once on the GPU and stay in HBM (the reference recomputes
-and re-uploads its tracing tables on every projector call,
-prj/src/prj_module.cu:380-398).
+bins and the z crossings along them are computed once on the GPU and stay in
+HBM (the reference recomputes and re-uploads its tracing tables on every
+projector call, prj/src/prj_module.cu:380-398). They take 4.3 GB a scanner and
+device: geometries of the same rays (spans, parameter sets) share them.
 """
 import ctypes as ct
 
