@@ -138,6 +138,20 @@ def check(rc, what=''):
         raise NipetError(f'{what}: {msg} (code {rc})')
 
 
+ENOMEM = -3  # NIPET_ENOMEM
+
+
+def with_room(call):
+    """Return code of ``call()``, called again where a device allocation of the
+    library failed and torch has given back the blocks that it only keeps."""
+    rc = call()
+    if rc == ENOMEM:
+        import torch
+        torch.cuda.empty_cache()
+        rc = call()
+    return rc
+
+
 def ptr(t):
     """Device (or host) address of a torch tensor / numpy array, or None."""
     if t is None:

@@ -39,6 +39,7 @@ void set_error(const char *fmt, ...) {
 }
 
 int hip_fail(hipError_t e, const char *what) {
+  (void)hipGetLastError();  // reported here, and not by the next launch's check
   set_error("HIP error %d (%s) in %s", (int)e, hipGetErrorString(e), what);
   return (e == hipErrorOutOfMemory) ? NIPET_ENOMEM : NIPET_EHIP;
 }

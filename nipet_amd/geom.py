@@ -48,7 +48,8 @@ class DeviceGeom:
         import torch
         h = ct.c_void_p()
         with torch.cuda.device(device):
-            _lib.check(_lib.lib().nipet_geom_create(ct.byref(d), ct.byref(h)), 'nipet_geom_create')
+            _lib.check(_lib.with_room(lambda: _lib.lib().nipet_geom_create(
+                ct.byref(d), ct.byref(h))), 'nipet_geom_create')
         self.handle = h
         self.naw = s2c.shape[0]
         self.nli = li2rng.shape[0]
