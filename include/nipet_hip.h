@@ -441,18 +441,17 @@ int nipet_philox4x32(const uint32_t *ctr, const uint32_t *key, uint32_t *out);
 #define NIPET_PROF_OTHER 5      /* small helper kernels */
 #define NIPET_PROF_BPRJ_PAIR 6  /* two-image BP of nipet_osem_subset_sens */
 int nipet_prof_enable(int on);
-/* Largest replicate sub-batch (4, 2 or 1) that one FP (kernel =
- * NIPET_PROF_FPRJ) or BP (NIPET_PROF_BPRJ) launch covers in the batched entry
- * points; batches are split greedily into sub-batches of at most that width.
- * Process-wide; set by the autotuner (no counterpart in the reference, whose
- * projectors take one image). */
+/* Replicate sub-batch width (4, 2 or 1) of the FP (kernel = NIPET_PROF_FPRJ) or
+ * BP (NIPET_PROF_BPRJ) in the batched entry points: with 4 or 2 a launch covers
+ * two images (the last of an odd batch one), with 1 one. Process-wide; set by the
+ * autotuner (no counterpart in the reference, whose projectors take one image). */
 int nipet_tune_set(int kernel, int width);
 int nipet_tune_get(int kernel, int *width);
 /* Run-length setting of the back projector at sub-batch width `width` (1, 2 or
  * 4): 8 or 6; 4 or 6; 6 or 4. Kept and reported; the back projector gives every
- * wave one run, whatever the setting. nipet_tune_get_run
- * also returns the other compiled length in *alt (may be NULL). No counterpart
- * in the reference (its ray blocks are fixed at compile time). */
+ * wave one run, whatever the setting. nipet_tune_get_run also returns the other
+ * of the two in *alt (may be NULL). No counterpart in the reference (its ray
+ * blocks are fixed at compile time). */
 int nipet_tune_set_run(int width, int spw);
 int nipet_tune_get_run(int width, int *spw, int *alt);
 int nipet_prof_reset(void);

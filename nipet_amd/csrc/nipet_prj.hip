@@ -1615,9 +1615,8 @@ static void launch_osem_update(float *img, const float *b, const float *sens, co
 
 using namespace nipet;
 
-// Launch a projector over nb replicates as sub-batches of 4, 2 and 1.
-// Largest replicate sub-batch per kernel instance (4, 2 or 1), set by the
-// autotuner through nipet_tune_set; process-wide.
+// Replicate sub-batch width (nipet_tune_set): 4 and 2 launch a projector over two
+// images at a time, 1 over one; process-wide.
 static std::atomic<int> g_width_fp{4}, g_width_bp{4};
 // Run lengths of nipet_tune_set_run: kept and reported; the back projector
 // now gives every wave one run.

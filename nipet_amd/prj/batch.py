@@ -37,7 +37,7 @@ FRAMES24 = ([(10 * i, 10 * i + 10) for i in range(14)] +
             [(200 + 20 * i, 220 + 20 * i) for i in range(5)] +
             [(300, 600)])
 
-GROUP = 4  # replicates per contiguous group (the widest kernel instance)
+GROUP = 4  # replicates per contiguous group (two pairs a launch of the projectors)
 
 
 def _torch():
@@ -49,13 +49,13 @@ _TUNED = {}
 
 
 def autotune(state, widths=(4, 2, 1), repeats=2, probe=4):
-    """Time the emission FP and the BP kernels on the first subset of
-    ``state`` (an ``OsemBatch``) over a probe batch of min(nb, ``probe``)
-    replicates, and keep the fastest shape per kernel: the FP sub-batch width,
-    and the BP sub-batch width together with its run length (segments per
-    wave run, kept as a setting: the kernel gives every wave one run). Results are cached
-    per (geometry, subset size) for the process. Returns {'fprj': w, 'bprj': w,
-    'bprj_run': {w: segments}, 'ms': {(kernel, w[, run]): ms per image}}."""
+    """Time the emission FP and the BP on the first subset of ``state`` (an
+    ``OsemBatch``), for a batch of min(nb, ``probe``) images as the state's own
+    lie, and keep the faster sub-batch width of each: images are projected in
+    pairs (width 2 or more) or one by one, so widths with the same launches as an
+    earlier one are not timed again. Results are cached per (geometry, subset
+    size) for the process. Returns {'fprj': w, 'bprj': w, 'bprj_run': {w: run
+    length in force}, 'ms': {(kernel, w[, run]): ms per image}}."""
     import ctypes as ct
     torch = _torch()
     L = _lib.lib()
@@ -64,8 +64,6 @@ def autotune(state, widths=(4, 2, 1), repeats=2, probe=4):
         res = _TUNED[key]
         _lib.check(L.nipet_tune_set(_lib.PROF_FPRJ, res['fprj']), 'nipet_tune_set')
         _lib.check(L.nipet_tune_set(_lib.PROF_BPRJ, res['bprj']), 'nipet_tune_set')
-        for w, run in res['bprj_run'].items():
-            _lib.check(L.nipet_tune_set_run(w, run), 'nipet_tune_set_run')
         return res
     st = _lib.stream_handle()
     subs = state.subsets[0]
@@ -74,9 +72,15 @@ def autotune(state, widths=(4, 2, 1), repeats=2, probe=4):
     img = torch.ones((320, 320, 127, nb), dtype=torch.float32, device='cuda')
     sino = torch.empty((nprj, state.geom.nsn, nb), dtype=torch.float32, device='cuda')
     bimg = torch.empty_like(img)
-    res = {'ms': {}, 'bprj_run': {}}
 
-    def timed(launch, n):
+    def run_length(w):
+        cur = ct.c_int()
+        _lib.check(L.nipet_tune_get_run(int(w), ct.byref(cur), None), 'tune_get_run')
+        return cur.value
+
+    res = {'ms': {}, 'bprj_run': {int(w): run_length(w) for w in widths}}
+
+    def timed(launch):
         launch()
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         e0.record()
@@ -84,47 +88,30 @@ def autotune(state, widths=(4, 2, 1), repeats=2, probe=4):
             launch()
         e1.record()
         e1.synchronize()
-        return e0.elapsed_time(e1) / repeats / n
+        return e0.elapsed_time(e1) / repeats / nb
 
-    def fprj(n):
-        return lambda: _lib.check(L.nipet_fprj_b(state.geom.handle, _lib.ptr(sino), _lib.ptr(img),
-                                                 _lib.ptr(subs), nprj, n, 0, st), 'nipet_fprj_b')
+    def fprj():
+        _lib.check(L.nipet_fprj_b(state.geom.handle, _lib.ptr(sino), _lib.ptr(img),
+                                  _lib.ptr(subs), nprj, nb, 0, st), 'nipet_fprj_b')
 
-    def bprj(n):
-        def launch():
-            with _lib.scratch(state.scratch):
-                _lib.check(L.nipet_bprj_b(state.geom.handle, _lib.ptr(bimg), _lib.ptr(sino),
-                                          _lib.ptr(subs), nprj, n, st), 'nipet_bprj_b')
-        return launch
-    best = None
-    for w in widths:
-        n = min(w, nb)
-        _lib.check(L.nipet_tune_set(_lib.PROF_FPRJ, int(w)), 'nipet_tune_set')
-        ms = timed(fprj(n), n)
-        res['ms'][('fprj', w)] = ms
-        if best is None or ms < best[1]:
-            best = (w, ms)
-    _lib.check(L.nipet_tune_set(_lib.PROF_FPRJ, best[0]), 'nipet_tune_set')
-    res['fprj'] = best[0]
-    best = None
-    for w in widths:
-        n = min(w, nb)
-        _lib.check(L.nipet_tune_set(_lib.PROF_BPRJ, int(w)), 'nipet_tune_set')
-        cur, alt = ct.c_int(), ct.c_int()
-        _lib.check(L.nipet_tune_get_run(int(w), ct.byref(cur), ct.byref(alt)), 'tune_get_run')
-        wbest = None
-        for run in (cur.value, alt.value):
-            _lib.check(L.nipet_tune_set_run(int(w), run), 'nipet_tune_set_run')
-            ms = timed(bprj(n), n)
-            res['ms'][('bprj', w, run)] = ms
-            if wbest is None or ms < wbest[1]:
-                wbest = (run, ms)
-        _lib.check(L.nipet_tune_set_run(int(w), wbest[0]), 'nipet_tune_set_run')
-        res['bprj_run'][int(w)] = wbest[0]
-        if best is None or wbest[1] < best[1]:
-            best = (w, wbest[1])
-    _lib.check(L.nipet_tune_set(_lib.PROF_BPRJ, best[0]), 'nipet_tune_set')
-    res['bprj'] = best[0]
+    def bprj():
+        with _lib.scratch(state.scratch):
+            _lib.check(L.nipet_bprj_b(state.geom.handle, _lib.ptr(bimg), _lib.ptr(sino),
+                                      _lib.ptr(subs), nprj, nb, st), 'nipet_bprj_b')
+
+    for name, kernel, launch in (('fprj', _lib.PROF_FPRJ, fprj), ('bprj', _lib.PROF_BPRJ, bprj)):
+        best, seen = None, set()
+        for w in widths:
+            if min(w, nb, 2) in seen:
+                continue
+            seen.add(min(w, nb, 2))
+            _lib.check(L.nipet_tune_set(kernel, int(w)), 'nipet_tune_set')
+            ms = timed(launch)
+            res['ms'][(name, w) if name == 'fprj' else (name, w, res['bprj_run'][int(w)])] = ms
+            if best is None or ms < best[1]:
+                best = (w, ms)
+        _lib.check(L.nipet_tune_set(kernel, best[0]), 'nipet_tune_set')
+        res[name] = best[0]
     _TUNED[key] = res
     return res
 
