@@ -1017,7 +1017,7 @@ template <int NB>
 constexpr int bp_threads() {
   return 512 * NB;
 }
-constexpr float BP_SNAP = 0x1p-45f, BP_FAINT = 0x1p-21f, BP_HUGE = 0x1p120f;
+constexpr float BP_SNAP = 0x1p-45f, BP_FAINT = 0x1p-23f, BP_HUGE = 0x1p120f;
 
 //
 // img: the image [voxel][nbt] (atomics, zeroed before), or with STAGED the

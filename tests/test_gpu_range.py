@@ -56,7 +56,8 @@ def rays(torch, geom, n, bright, faint, seed):
     return torch.where(big > 0, big, y), big
 
 
-@pytest.mark.parametrize('bright,faint', [(1e6, 1e-12), (3.4e38, 1.0), (1.0, 1e-6), (1e30, 1e-30)])
+@pytest.mark.parametrize('bright,faint', [(1e6, 1e-12), (3.4e38, 1.0), (1.0, 1e-6), (1.0, 3e-7),
+                                          (1.0, 1e-7), (1e30, 1e-30)])
 def test_back_projection_small_beside_large(torch, lib, params, bright, faint):
     """Float atomics against the FP64 oracle."""
     from nipet_amd.geom import get_geom
