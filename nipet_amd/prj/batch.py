@@ -18,14 +18,14 @@ normalisation (hence the 14 sensitivity images) run as one batch:
 * replicates are stored in contiguous groups of ``GROUP`` ([group][voxel][4],
   prompts [group][bin][837][4]): a kernel launch covers one group, so every
   cache line it touches holds only that group's replicates;
-* the replicate sub-batch width of the FP and BP kernels (4, 2 or 1 images per
-  launch), and the BP's run length at each width, are picked by timing the
-  kernels on the problem's own geometry and group size (``autotune``).
+* the replicate sub-batch width of the FP and BP kernels (pairs or single images
+  per launch) is picked by timing them on the problem's own geometry and group
+  (``autotune``).
 """
 import numpy as np
 
 from .. import _lib
-from .osem import OsemBatch, osem_iteration_batch, osem_prepare_batch
+from .osem import OsemBatch, osem_iteration_batch, osem_prepare_batch, osem_subset_batch
 
 __all__ = ['GROUP', 'autotune', 'prepare_groups', 'OsemGraph', 'bootstrap_prompts',
            'frame_prompts', 'bootstrap_osem', 'frames_osem', 'FRAMES24', 'replicates_and_frames']
@@ -165,15 +165,18 @@ class OsemGraph:
         self.imgs = [torch.ones((320, 320, 127, st.nb), dtype=torch.float32, device='cuda')
                      for st in states]
         _lib.check(_lib.lib().nipet_prof_enable(0), 'nipet_prof_enable')
-        # load every kernel instance before capture: one subset update over a
-        # single transaxial bin per group (the images are reset before each run)
+        # load every kernel instance before capture: the captured updates of the
+        # shortest and the longest subset (few bins are not staged) of every kind
+        # of group (the images are reset before each run)
+        seen = set()
         for st, img in zip(states, self.imgs):
-            first = st.subsets[0][:1].contiguous()
-            _lib.check(_lib.lib().nipet_osem_subset_b(
-                st.geom.handle, _lib.ptr(img), _lib.ptr(st.prompts), _lib.ptr(st.rho),
-                int(st.rho_per_rep), _lib.ptr(st.sens[0]), 0, _lib.ptr(st.mask), None,
-                _lib.ptr(first), 1, st.nb, _lib.ptr(st.work_sino), _lib.ptr(st.work_img),
-                _lib.stream_handle()), 'nipet_osem_subset_b')
+            kind = (st.nb, st.krnl is None, st.scratch is None)
+            if kind in seen:
+                continue
+            seen.add(kind)
+            by_len = sorted(range(len(st.subsets)), key=lambda k: len(st.subsets[k]))
+            for k in {by_len[0], by_len[-1]}:
+                osem_subset_batch(st, img, k)
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(self.graph):

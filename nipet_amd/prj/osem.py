@@ -424,15 +424,18 @@ def osem_prepare_batch(scanner_params, prompts, asng, nsng, rsng=None, ssng=None
 
 def osem_iteration_batch(state, img, first_full=True):
     """One OSEM iteration of all nb images; windows as ``osem_iteration``."""
-    with _lib.scratch(state.scratch):
-        _subsets_batch(state, img, first_full)
+    for k in range(len(state.subsets)):
+        osem_subset_batch(state, img, k, windowed=not (k == 0 and first_full))
 
 
-def _subsets_batch(state, img, first_full):
+def osem_subset_batch(state, img, k, windowed=True):
+    """The update of subset ``k`` for all nb images, along the mask's segment
+    windows or whole rays."""
     st = _lib.stream_handle()
     L = _lib.lib()
-    for k, subs in enumerate(state.subsets):
-        win = None if (k == 0 and first_full) else _lib.ptr(state.win)
+    subs = state.subsets[k]
+    win = _lib.ptr(state.win) if windowed else None
+    with _lib.scratch(state.scratch):
         if state.krnl is not None:
             _lib.check(L.nipet_osem_subset_rm_b(
                 state.geom.handle, _lib.ptr(img), _lib.ptr(state.prompts), _lib.ptr(state.rho),
@@ -440,7 +443,7 @@ def _subsets_batch(state, img, first_full):
                 _lib.ptr(subs), len(subs), state.nb, state.krnl.ctypes.data,
                 _lib.ptr(state.work_sino), _lib.ptr(state.work_img), _lib.ptr(state.work_img2),
                 st), 'nipet_osem_subset_rm_b')
-            continue
+            return
         _lib.check(L.nipet_osem_subset_b(
             state.geom.handle, _lib.ptr(img), _lib.ptr(state.prompts), _lib.ptr(state.rho),
             int(state.rho_per_rep), _lib.ptr(state.sens[k]), 0, _lib.ptr(state.mask), win,
