@@ -147,6 +147,7 @@ class OsemState:
         self._pair = None
         # staged back projections (two images while sensitivities are pending)
         self.scratch = _lib.bprj_scratch(geom, self.nprj, 2 if self.pending else 1)
+        self._two = bool(self.pending)
 
     @property
     def sens(self):
@@ -158,7 +159,20 @@ class OsemState:
             sensitivity(self.geom, self.an, self.subsets[k], out=self._sens[k],
                         scratch=self.scratch)
         self.pending.clear()
+        self.settle()
         return self._sens
+
+    def settle(self):
+        """Once no sensitivity image is pending: scratch for one image in the
+        place of that for two."""
+        if self.pending or not self._two:
+            return
+        self._two = False
+        if self.scratch is not None:
+            # (the current stream may still use it)
+            self.scratch.record_stream(_torch().cuda.current_stream())
+            self.scratch = None
+        self.scratch = _lib.bprj_scratch(self.geom, self.nprj)
 
     def pair_work(self):
         """Work buffers of the two-image first update (allocated while subsets
@@ -275,6 +289,7 @@ def osem_iteration(state, img, first_full=True):
     False (an image already masked by an earlier update)."""
     with _lib.scratch(state.scratch):
         _subsets(state, img, first_full)
+    state.settle()
 
 
 def _subsets(state, img, first_full):
