@@ -97,9 +97,9 @@ int nipet_fprj(const NipetGeom *g, float *sino, const float *img, const int32_t 
  * a device buffer, 256-byte aligned, that every later call of this thread may
  * overwrite in its stream's order, until it is replaced or taken back with (NULL,
  * 0). With at least nipet_bprj_scratch bytes the per-segment sums are staged
- * there and gathered by voxel column (a fixed order of additions); with less, in
- * several passes; without, or for few bins, they are float atomics into the
- * image. nipet_bprj_scratch: bytes for nprj bins of nb images (0: none used). */
+ * there and gathered by voxel column (a fixed order of additions, except among
+ * rows of one and the same bin); with less, in several passes; without, or for
+ * few bins, they are float atomics into the image. nipet_bprj_scratch: bytes for nprj bins of nb images (0: none used). */
 int64_t nipet_bprj_scratch(const NipetGeom *g, int nprj, int nb);
 int nipet_scratch_set(void *buf, int64_t bytes);
 

@@ -1315,7 +1315,8 @@ constexpr int BP_NAW = 1 << 17;
 
 // Rows of the launch by transaxial bin, for k_bp_gather. bits: the bins that
 // have rows; head[aw].x = last row of bin aw, head[aw].y = its written segments,
-// first | count << 16; next[row] = the row before it of the same bin, or -1.
+// first | count << 16; next[row] = another row of the same bin, or -1 (in no
+// fixed order: rows of a bin that is listed more than once are added in any).
 __global__ void k_bp_clear(int2 *head, uint32_t *bits, int naw) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < naw) head[i].x = -1;
@@ -1334,8 +1335,8 @@ __global__ void k_bp_link(int2 *head, uint32_t *bits, int32_t *next, const int32
 }
 
 // Sums the staged rows of every voxel column: one wave per column, which walks
-// the column's segments of all bins (GeomView::col_ent, ascending, so the sum's
-// order is fixed) and adds the rows of the bins in this launch, 512 bytes an
+// the column's segments of all bins (GeomView::col_ent, ascending, so the order
+// of the bins is fixed) and adds the rows of the bins in this launch, 512 bytes an
 // image each. add: to the image (later passes) rather than over it.
 // A column has a few hundred entries, of which one in 14 (a subset) has a row:
 // 64 BP_GE entries are read together and sieved with the bins' bits in LDS;
@@ -1629,7 +1630,7 @@ static thread_local struct {
   int64_t bytes;
 } t_scratch = {nullptr, 0};
 
-// Rows at the largest (bins per pass, 1.2 GB an image), and bins from which
+// Rows at the largest (bins per pass, 1.7 GB an image at 406 segments), and bins from which
 // staging pays: one image's back projection with float atomics / staged took
 // 0.204 / 0.222 ms for 1,024 bins, 0.295 / 0.293 for 1,536, 0.359 / 0.350 for
 // 2,048 and 0.742 / 0.673 for a subset of 4,893 (the columns' walk costs the same
