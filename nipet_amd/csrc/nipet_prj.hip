@@ -138,7 +138,7 @@ __device__ inline double rdlane(double v, int l) {
 //   C_{2 d - w_end + 2 r0}(t_end) - sum_w [C_p - C_{p + 1}](t_w), p = 2 d - w - 1 + 2 r0.
 // The work is therefore one LDS read per z crossing (about 1.8 d per LOR, 37
 // on average), not one per voxel segment (272 on average): a subset of 4,894
-// bins takes 0.50 ms against 0.95 by segments, all 68,516 bins 6.7 against
+// bins takes 0.49 ms against 0.95 by segments, all 68,516 bins 6.7 against
 // 12.6. VALU, scalar unit and LDS are each at 0.6 of their limits: what is left
 // is waves waiting for their turn at all three.
 //  - Rows E[j][p] = (C_p - C_{p + 1}) at the start of segment j, a float64
@@ -604,9 +604,10 @@ __global__ __launch_bounds__(FZ_THREADS, NB == 1 ? 8 : 4) void k_fprj(
 // ---------------------------------------------------------------------------
 // Forward projection by segments (nipet_fprj_seg; MODE 0: emission, 1:
 // attenuation factors): every LOR visits every segment of the bin, in float32.
-// The differentiable projectors' forward passes keep it: their likelihood is a
+// The differentiable projectors' forward passes use it: their likelihood is a
 // float64 number made of these float32 values, and it stays the same bit for
-// bit. (k_fprj is 1.7 times faster and differs by 5e-8.)
+// bit. (k_fprj takes 0.49 ms a subset instead of 1.04, and differs by 5e-8: 4.9e-8
+// from the exact values instead of 5.6e-8.)
 //
 // Lanes are groups of G LORs of one ring difference.
 // LOR (d, r0 + k) lies exactly 2k planes above LOR (d, r0) along the whole ray
@@ -1011,8 +1012,10 @@ __global__ __launch_bounds__(256) void k_seg_window(GeomView g, const uint8_t *_
 //  - Output: with STAGED every segment's plane sums go to the segment's own row
 //    of a scratch buffer (512 bytes an image) and k_bp_gather adds the rows of
 //    each voxel column, else float atomics to the image.
-// Bound by vector issue (82 % of the cycles, 8 waves per SIMD): 0.40 ms a subset
-// for one image, 0.68 for two (with 512 threads, 4 waves per SIMD, 0.82).
+// Bound by vector issue (80 % of the cycles, 8 waves per SIMD): 0.40 ms a subset
+// for one image, 0.67 for two (with 512 threads, 4 waves per SIMD, 0.82), of which
+// the look for small sums is 0.5 %; where every bin has some, 2.7 ms with the
+// gather.
 template <int NB>
 constexpr int bp_threads() {
   return 512 * NB;

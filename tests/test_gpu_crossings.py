@@ -4,7 +4,7 @@ odd and strided batches, segment windows and single bins.
 
 Tolerance: the parity bar of the projectors, 1e-5 of each value with values
 below 1e-6 of the largest held to that floor; the kernel rounds to float32
-(6e-8) and keeps a boundary's distance into its segment in float32 (7e-9 cm)."""
+(6e-8) and keeps a boundary's distance into its segment to 2^-32 of it."""
 import ctypes as ct
 
 import numpy as np
